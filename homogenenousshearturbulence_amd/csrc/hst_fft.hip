@@ -345,7 +345,8 @@ __device__ __forceinline__ Cx<R> combined_product(int p, const Cx<R> &u, const C
 
 // ------------------------------------------------------------------ k_xpass
 
-// One (row, z point) line per group of T threads, G lines per block.
+// One (row, z point) line per group of T threads, G lines per block; for the
+// shortest lines (M = 6, 12), which k_xline does not take.
 // MODE 0: six products; 1: the round trip (u, v, w times factor); 2: CFL only.
 template <typename R, int M, int MODE>
 __global__ void __launch_bounds__((XCfg<R, M>::NT))
@@ -435,39 +436,67 @@ __global__ void __launch_bounds__((XCfg<R, M>::NT))
 
 // ------------------------------------------------------------------ k_xline
 
-// The x pass for power-of-two lengths M >= 64: T = M/8 threads per line,
-// E = 8 elements per thread; a block is one wavefront holding 64/T lines, or
-// at M = 1024 two wavefronts holding one line.  A
-// thread holds the elements t + T e (e < E) of a line in registers; the
-// Stockham stages exchange through LDS only between stages, and the last
-// stage of a transform leaves the elements t + T e in the registers of
-// thread t again, which is where the first stage of the next transform
-// reads them: the products are formed in registers between the inverse and
-// the forward transforms.  LDS lines are padded by one element per eight.
+// The x pass for lengths M = 2^a >= 16 and M = 3 2^a >= 24: T = M/8 threads
+// per line, E = 8 elements per thread.  A thread holds the elements t + T e
+// (e < E) of a line in registers; the Stockham stages exchange through LDS
+// only between stages, and the last stage of a transform leaves the elements
+// t + T e in the registers of thread t again, which is where the first stage
+// of the next transform reads them: the products are formed in registers
+// between the inverse and the forward transforms.  LDS lines are padded by
+// one element per eight.
+//
+// A line has TS lanes: T of them for M = 2^a, M/6 (so a power of two) for
+// M = 3 2^a, whose radix-8, 4 and 2 stages then leave a quarter of the lanes
+// idle while the radix-3 stage, the second one, takes them all.  A line of up
+// to 64 lanes so stays inside one wavefront and needs no block barrier between
+// its stages.  The lengths 3 2^a went through k_xpass before, which keeps the
+// velocities in LDS and passes every product through it: M = 192, 261 rows of
+// 384 lines, 1475 -> 663 us in FP64 and 762 -> 326 us in FP32; M = 96, 132 rows
+// of 192 lines, 171 -> 90 and 98 -> 55 us.  It is bound as the power-of-two lines
+// are: FP64 by LDS and its latency at two wavefronts a SIMD, FP32 by the vector
+// ALU.
 template <int M>
 struct XL {
+  static constexpr bool THREE = M % 3 == 0;
   static constexpr int T = M / 8;
-  static constexpr int E = M / T;
+  static constexpr int TS = THREE ? M / 6 : T;
+  static constexpr int E = 8;
   // lines per block: at least four neighbouring z points (a tile's four
   // points are one 128-byte run of the product buffer), a wavefront at least
-  static constexpr int LPB = 64 / T > 4 ? 64 / T : 4;
-  static constexpr int NTH = LPB * T;  // threads per block
+  static constexpr int LPB = 64 / TS > 4 ? 64 / TS : (TS > 128 ? 2 : 4);
+  static constexpr int NTH = LPB * TS;  // threads per block
   static constexpr int PL = M + M / 8;
   // kept x modes a line can have: nx + 1 <= 2 nxd / 3 (the 3/2 rule)
   static constexpr int NXS = 2 * M / 3 + 2;
 };
+constexpr bool xline_size(int M) { return M % 3 == 0 ? M >= 24 : M >= 16; }
+
+// The x pass's radices: those of the z lines for M = 2^a; for M = 3 2^a the
+// radix 3 comes second, so that the first and the last stage divide E.
+__host__ __device__ constexpr int xl_rest(int R, int i) {  // radix i of the rest R after 8 and 3
+  return R == 16 ? 4 : R <= 8 ? R : (i == 0 ? 8 : R / 8);
+}
+__host__ __device__ constexpr int xl_radix(int M, int st) {
+  if (M % 3) return radix_at(M, st);
+  const int first = M == 24 ? 4 : 8;
+  return st == 0 ? first : (st == 1 ? 3 : xl_rest(M / (3 * first), st - 2));
+}
+__host__ __device__ constexpr int xl_stages(int M) {
+  if (M % 3) return n_stages(M);
+  const int R = M / (M == 24 ? 12 : 24);
+  return 2 + (R > 8 ? 2 : 1);
+}
 
 __device__ __forceinline__ int padx(int p) { return p + (p >> 3); }
 
 // The exchange between two Stockham stages of a line: a line of up to 64
-// threads lives in one wavefront and in its own part of LDS, so the
+// lanes lives in one wavefront and in its own part of LDS, so the
 // wavefront need only wait for its own LDS traffic (the LDS serves a
 // wavefront's requests in order; the fences keep the compiler from moving
-// them across); the 1024-point lines span two wavefronts and take the
-// block's barrier.
+// them across); longer lines span wavefronts and take the block's barrier.
 template <int M>
 __device__ __forceinline__ void xl_sync() {
-  if constexpr (XL<M>::T <= 64) {
+  if constexpr (XL<M>::TS <= 64) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -483,76 +512,112 @@ __device__ __forceinline__ void xl_sync() {
 // neighbouring words (read as tw[n1 k2 S], a stage's lanes hit one bank).
 template <int M, int ST = 0, int S = 1>
 __host__ __device__ constexpr int xtw_off(int st) {
-  if constexpr (ST + 1 >= n_stages(M)) {
+  if constexpr (ST + 1 >= xl_stages(M)) {
     return 0;
   } else {
-    constexpr int RAD = radix_at(M, ST), Ls = M / (S * RAD);
+    constexpr int RAD = xl_radix(M, ST), Ls = M / (S * RAD);
     return st <= ST ? 0 : (RAD - 1) * Ls + xtw_off<M, ST + 1, S * RAD>(st);
   }
 }
 template <int M>
-__host__ __device__ constexpr int xtw_size() { return xtw_off<M>(n_stages(M)); }
+__host__ __device__ constexpr int xtw_size() { return xtw_off<M>(xl_stages(M)); }
 // the exponent n1 k2 S of entry i of the staged table
 template <int M, int ST = 0, int S = 1>
 __device__ __forceinline__ int xtw_exponent(int i) {
-  if constexpr (ST + 1 >= n_stages(M)) {
+  if constexpr (ST + 1 >= xl_stages(M)) {
     return 0;
   } else {
-    constexpr int RAD = radix_at(M, ST), Ls = M / (S * RAD), n = (RAD - 1) * Ls;
+    constexpr int RAD = xl_radix(M, ST), Ls = M / (S * RAD), n = (RAD - 1) * Ls;
     if (i < n) return (i % Ls) * (1 + i / Ls) * S;
     return xtw_exponent<M, ST + 1, S * RAD>(i - n);
   }
 }
 
+// One line's transform; act: the lane is one of the line's T (always, for
+// M = 2^a).  The lanes past T take part in the radix-3 stage alone.
 template <typename R, int M, int SIGN, int ST, int S>
-__device__ __forceinline__ void xl_fft(Cx<R> (&v)[XL<M>::E], Cx<R> *L, int t, const Cx<R> *__restrict__ tw) {
-  constexpr int T = XL<M>::T, E = XL<M>::E;
-  if constexpr (ST < n_stages(M)) {
-    constexpr int RAD = radix_at(M, ST);
+__device__ __forceinline__ void xl_fft(Cx<R> (&v)[XL<M>::E], Cx<R> *L, int t, bool act,
+                                       const Cx<R> *__restrict__ tw) {
+  constexpr int T = XL<M>::T, TS = XL<M>::TS, E = XL<M>::E;
+  if constexpr (ST < xl_stages(M)) {
+    constexpr int RAD = xl_radix(M, ST);
     constexpr int Ls = M / (S * RAD);
-    constexpr int NB = E / RAD;
     constexpr bool FIRST = (S == 1), LAST = (S * RAD == M);
-    Cx<R> c[NB][RAD];
+    constexpr int OFF = xtw_off<M>(ST);
+    if constexpr (RAD == 3) {
+      // M/3 butterflies, two for each of the line's TS = M/6 lanes
+      static_assert(!FIRST && !LAST && 6 * TS == M, "the radix-3 stage lies inside");
+      Cx<R> c[2][3];
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-      if constexpr (FIRST) {
+      for (int j = 0; j < 2; j++) {
+        const int b = t + TS * j, q = b % S, n1 = b / S;
 #pragma unroll
-        for (int n2 = 0; n2 < RAD; n2++) c[j][n2] = v[j + NB * n2];
-      } else {
-        const int b = t + T * j, q = b % S, n1 = b / S;
-#pragma unroll
-        for (int n2 = 0; n2 < RAD; n2++) c[j][n2] = L[padx(q + S * (n1 + Ls * n2))];
-      }
-    }
-    xl_sync<M>();  // every read of L done before it is written again
-#pragma unroll
-    for (int j = 0; j < NB; j++) {
-      dft<R, SIGN, RAD>(c[j]);
-      if constexpr (!LAST) {
-        const int b = t + T * j, n1 = b / S;
-        constexpr int OFF = xtw_off<M>(ST);
-#pragma unroll
-        for (int k2 = 1; k2 < RAD; k2++) {
-          Cx<R> w = tw[OFF + (k2 - 1) * Ls + n1];
-          if (SIGN > 0) w.y = -w.y;
-          c[j][k2] = c[j][k2] * w;
-        }
-      }
-    }
-    if constexpr (LAST) {
-#pragma unroll
-      for (int j = 0; j < NB; j++)
-#pragma unroll
-        for (int k2 = 0; k2 < RAD; k2++) v[j + NB * k2] = c[j][k2];
-    } else {
-#pragma unroll
-      for (int j = 0; j < NB; j++) {
-        const int b = t + T * j, q = b % S, n1 = b / S;
-#pragma unroll
-        for (int k2 = 0; k2 < RAD; k2++) L[padx(q + S * k2 + S * RAD * n1)] = c[j][k2];
+        for (int n2 = 0; n2 < 3; n2++) c[j][n2] = L[padx(q + S * (n1 + Ls * n2))];
       }
       xl_sync<M>();
-      xl_fft<R, M, SIGN, ST + 1, S * RAD>(v, L, t, tw);
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const int b = t + TS * j, q = b % S, n1 = b / S;
+        dft<R, SIGN, 3>(c[j]);
+        L[padx(q + S * 3 * n1)] = c[j][0];
+#pragma unroll
+        for (int k2 = 1; k2 < 3; k2++) {
+          Cx<R> w = tw[OFF + (k2 - 1) * Ls + n1];
+          if (SIGN > 0) w.y = -w.y;
+          L[padx(q + S * k2 + S * 3 * n1)] = c[j][k2] * w;
+        }
+      }
+      xl_sync<M>();
+      xl_fft<R, M, SIGN, ST + 1, S * RAD>(v, L, t, act, tw);
+    } else {
+      constexpr int NB = E / RAD;
+      Cx<R> c[NB][RAD];
+      if (act) {
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+          if constexpr (FIRST) {
+#pragma unroll
+            for (int n2 = 0; n2 < RAD; n2++) c[j][n2] = v[j + NB * n2];
+          } else {
+            const int b = t + T * j, q = b % S, n1 = b / S;
+#pragma unroll
+            for (int n2 = 0; n2 < RAD; n2++) c[j][n2] = L[padx(q + S * (n1 + Ls * n2))];
+          }
+        }
+      }
+      xl_sync<M>();  // every read of L done before it is written again
+      if (act) {
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+          dft<R, SIGN, RAD>(c[j]);
+          if constexpr (!LAST) {
+            const int b = t + T * j, n1 = b / S;
+#pragma unroll
+            for (int k2 = 1; k2 < RAD; k2++) {
+              Cx<R> w = tw[OFF + (k2 - 1) * Ls + n1];
+              if (SIGN > 0) w.y = -w.y;
+              c[j][k2] = c[j][k2] * w;
+            }
+          }
+        }
+        if constexpr (LAST) {
+#pragma unroll
+          for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int k2 = 0; k2 < RAD; k2++) v[j + NB * k2] = c[j][k2];
+        } else {
+#pragma unroll
+          for (int j = 0; j < NB; j++) {
+            const int b = t + T * j, q = b % S, n1 = b / S;
+#pragma unroll
+            for (int k2 = 0; k2 < RAD; k2++) L[padx(q + S * k2 + S * RAD * n1)] = c[j][k2];
+          }
+        }
+      }
+      if constexpr (!LAST) {
+        xl_sync<M>();
+        xl_fft<R, M, SIGN, ST + 1, S * RAD>(v, L, t, act, tw);
+      }
     }
   }
 }
@@ -574,7 +639,7 @@ __device__ __forceinline__ void xl_c2r_load(Cx<R> (&dst)[XL<M>::E], const Cx<R> 
     b[e] = Cx<R>{(R)0, (R)0};
     if (ok && k <= nx) a[e] = src[hoff<R>(NZD, NXp, zp, k)];
     if (ok && k > 0 && M - k <= nx) b[e] = src[hoff<R>(NZD, NXp, zp, M - k)];
-    ep[e] = twh[k];
+    ep[e] = twh[min(k, M - 1)];  // (a lane without elements reads the last)
   }
 #pragma unroll
   for (int e = 0; e < E; e++) {
@@ -589,12 +654,13 @@ __device__ __forceinline__ void xl_c2r_load(Cx<R> (&dst)[XL<M>::E], const Cx<R> 
 // occupancy floor (wavefronts per SIMD): the FP64 lines fit in 256 VGPRs (two
 // wavefronts per SIMD) with a few bytes of spill instead of taking one; the
 // FP32 lines are bound by the vector ALU and run 4 % faster at four
-// wavefronts with 36 bytes of spill than at three without
-#ifndef XLINE_F32_WAVES
-#define XLINE_F32_WAVES 4
-#endif
+// wavefronts with 36 bytes of spill than at three without.  With the radix-3
+// stage's butterflies beside the elements four wavefronts spill 25 to 39
+// registers: three run 1.2 to 1.3 times faster (M = 192 420 -> 326 us, M = 384
+// 2076 -> 1590 us at 261 rows), but for the blocks of eight wavefronts of
+// M >= 768, of which only one would fit a CU (170 us at four, 190 at three).
 template <typename R, int M>
-constexpr int xline_min_waves() { return sizeof(R) == 8 ? 2 : XLINE_F32_WAVES; }
+constexpr int xline_min_waves() { return sizeof(R) == 8 ? 2 : (M % 3 == 0 && M < 768 ? 3 : 4); }
 
 template <typename R, int M, int MODE>
 __global__ void __launch_bounds__(XL<M>::NTH, (xline_min_waves<R, M>()))
@@ -612,7 +678,8 @@ __global__ void __launch_bounds__(XL<M>::NTH, (xline_min_waves<R, M>()))
   __shared__ Cx<R> twhl[M];
   lds_fill<M, NTH>(twhl, [&](int k) { return twh[k]; });
   __syncthreads();
-  const int g = threadIdx.x / T, t = threadIdx.x % T;
+  const int g = threadIdx.x / XL<M>::TS, t = threadIdx.x % XL<M>::TS;
+  const bool act = XL<M>::TS == T || t < T;  // a lane that holds elements
   const int NZD = D.nzd, nx = D.nx;
   // tiled Hv: neighbouring z points share cache lines, so neighbouring
   // blocks stay on one XCD (one L2)
@@ -627,17 +694,17 @@ __global__ void __launch_bounds__(XL<M>::NTH, (xline_min_waves<R, M>()))
   Cx<R> u[E], v[E], w[E];
   // C2R pre-processing of u, v, w straight from the x modes in HBM
   const size_t plane = (size_t)NZD * D.NXp;
-  xl_c2r_load<R, M>(u, Hv + ((size_t)0 * nrows + rowc) * plane, NZD, D.NXp, zp, ok, t, nx, twh);
-  xl_c2r_load<R, M>(v, Hv + ((size_t)1 * nrows + rowc) * plane, NZD, D.NXp, zp, ok, t, nx, twh);
-  xl_c2r_load<R, M>(w, Hv + ((size_t)2 * nrows + rowc) * plane, NZD, D.NXp, zp, ok, t, nx, twh);
-  xl_fft<R, M, +1, 0, 1>(u, L, t, twl);
-  xl_fft<R, M, +1, 0, 1>(v, L, t, twl);
-  xl_fft<R, M, +1, 0, 1>(w, L, t, twl);
+  xl_c2r_load<R, M>(u, Hv + ((size_t)0 * nrows + rowc) * plane, NZD, D.NXp, zp, ok && act, t, nx, twh);
+  xl_c2r_load<R, M>(v, Hv + ((size_t)1 * nrows + rowc) * plane, NZD, D.NXp, zp, ok && act, t, nx, twh);
+  xl_c2r_load<R, M>(w, Hv + ((size_t)2 * nrows + rowc) * plane, NZD, D.NXp, zp, ok && act, t, nx, twh);
+  xl_fft<R, M, +1, 0, 1>(u, L, t, act, twl);
+  xl_fft<R, M, +1, 0, 1>(v, L, t, act, twl);
+  xl_fft<R, M, +1, 0, 1>(w, L, t, act, twl);
   // u[e] = x(2k) + i x(2k+1) at k = t + T e
   if (want_cfl) {
     double cm = 0.0;
     const int iy = row0 + rowc - 2;
-    if (ok && iy >= 0 && iy < D.ny) {
+    if (ok && act && iy >= 0 && iy < D.ny) {
       const double idx = 1.0 / D.dx, idy = 1.0 / dyl[iy], idz = 1.0 / D.dz;
 #pragma unroll
       for (int e = 0; e < E; e++) {
@@ -684,16 +751,17 @@ __global__ void __launch_bounds__(XL<M>::NTH, (xline_min_waves<R, M>()))
         z[e] = Cx<R>{a.x * b.x * factor, a.y * b.y * factor};
       }
     }
-    xl_fft<R, M, -1, 0, 1>(z, L, t, twl);
+    xl_fft<R, M, -1, 0, 1>(z, L, t, act, twl);
     // R2C post-processing needs Z(k) and Z(M - k)
 #pragma unroll
-    for (int e = 0; e < E; e++) L[padx(t + T * e)] = z[e];
+    for (int e = 0; e < E; e++)
+      if (act) L[padx(t + T * e)] = z[e];
     xl_sync<M>();
 #pragma unroll
     for (int e = 0; e < E; e++) {
       const int k = t + T * e;
-      if (k <= nx) {
-        const Cx<R> Z = z[e], Zc = conj(L[padx((M - k) & (M - 1))]);
+      if (act && k <= nx) {
+        const Cx<R> Z = z[e], Zc = conj(L[padx(k == 0 ? 0 : M - k)]);
         const Cx<R> ep = twhl[k];  // exp(-i pi k / M)
         z[e] = (Z + Zc) - mul_i(ep * (Z - Zc));
       }
@@ -705,7 +773,7 @@ __global__ void __launch_bounds__(XL<M>::NTH, (xline_min_waves<R, M>()))
 #pragma unroll
     for (int e = 0; e < E; e++) {
       const int k = t + T * e;
-      if (k <= nx) L[k] = z[e];
+      if (act && k <= nx) L[k] = z[e];
     }
     __syncthreads();
     // the block's lines to the tiles: consecutive threads take the lines of
@@ -754,7 +822,7 @@ static int run_zfft(const Dims &D, int np, const void *Hp, void *P0, size_t pstr
 template <typename R, int M>
 static int run_xpass(const Dims &D, int mode, const void *Hv, void *Hp, int row0, int nrows, const Tables<R> &tb,
                      const double *dyl, double *cfl_part, int want_cfl, int *n_part, hipStream_t s) {
-  if constexpr ((M & (M - 1)) == 0 && M >= 64) {
+  if constexpr (xline_size(M)) {
     typedef XL<M> C;
     if (D.nx + 1 > C::NXS) return hipErrorInvalidValue;
     const int lines = D.nzd * nrows;
