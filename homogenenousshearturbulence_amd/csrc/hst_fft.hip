@@ -639,7 +639,7 @@ __device__ __forceinline__ void xl_c2r_load(Cx<R> (&dst)[XL<M>::E], const Cx<R> 
     b[e] = Cx<R>{(R)0, (R)0};
     if (ok && k <= nx) a[e] = src[hoff<R>(NZD, NXp, zp, k)];
     if (ok && k > 0 && M - k <= nx) b[e] = src[hoff<R>(NZD, NXp, zp, M - k)];
-    ep[e] = twh[min(k, M - 1)];  // (a lane without elements reads the last)
+    ep[e] = twh[XL<M>::THREE ? min(k, M - 1) : k];  // (a lane without elements reads the last)
   }
 #pragma unroll
   for (int e = 0; e < E; e++) {
@@ -752,7 +752,8 @@ __global__ void __launch_bounds__(XL<M>::NTH, (xline_min_waves<R, M>()))
       }
     }
     xl_fft<R, M, -1, 0, 1>(z, L, t, act, twl);
-    // R2C post-processing needs Z(k) and Z(M - k)
+    // R2C post-processing needs Z(k) and Z(M - k), Z(M) = Z(0) (for M = 2^a
+    // the mask, not a select: the select's registers spill in FP32, 16 % slower)
 #pragma unroll
     for (int e = 0; e < E; e++)
       if (act) L[padx(t + T * e)] = z[e];
@@ -761,7 +762,7 @@ __global__ void __launch_bounds__(XL<M>::NTH, (xline_min_waves<R, M>()))
     for (int e = 0; e < E; e++) {
       const int k = t + T * e;
       if (act && k <= nx) {
-        const Cx<R> Z = z[e], Zc = conj(L[padx(k == 0 ? 0 : M - k)]);
+        const Cx<R> Z = z[e], Zc = conj(L[padx(XL<M>::THREE ? (k == 0 ? 0 : M - k) : (M - k) & (M - 1))]);
         const Cx<R> ep = twhl[k];  // exp(-i pi k / M)
         z[e] = (Z + Zc) - mul_i(ep * (Z - Zc));
       }
