@@ -343,6 +343,21 @@ __device__ __forceinline__ Cx<R> combined_product(int p, const Cx<R> &u, const C
   }
 }
 
+// The six products uu, vv, ww, uv, vw, uw, each times factor, on the even (x)
+// and odd (y) points of a line.  A switch on p, not selects of the arrays by p:
+// the selects left the six-product x pass with 50 to 84 spilled registers.
+template <typename R>
+__device__ __forceinline__ Cx<R> plain_product(int p, const Cx<R> &u, const Cx<R> &v, const Cx<R> &w, R factor) {
+  switch (p) {
+    case 0: return Cx<R>{u.x * u.x * factor, u.y * u.y * factor};
+    case 1: return Cx<R>{v.x * v.x * factor, v.y * v.y * factor};
+    case 2: return Cx<R>{w.x * w.x * factor, w.y * w.y * factor};
+    case 3: return Cx<R>{u.x * v.x * factor, u.y * v.y * factor};
+    case 4: return Cx<R>{v.x * w.x * factor, v.y * w.y * factor};
+    default: return Cx<R>{u.x * w.x * factor, u.y * w.y * factor};
+  }
+}
+
 // ------------------------------------------------------------------ k_xpass
 
 // One (row, z point) line per group of T threads, G lines per block; for the
@@ -740,16 +755,9 @@ __global__ void __launch_bounds__(XL<M>::NTH, (xline_min_waves<R, M>()))
     Cx<R> z[E];
 #pragma unroll
     for (int e = 0; e < E; e++) {
-      if constexpr (MODE == 1) {
-        const Cx<R> a = (p == 0 ? u[e] : (p == 1 ? v[e] : w[e]));
-        z[e] = Cx<R>{a.x * factor, a.y * factor};
-      } else if constexpr (MODE == 3) {
-        z[e] = combined_product<R>(p, u[e], v[e], w[e], factor);
-      } else {
-        const Cx<R> a = (p == 0 || p == 3 || p == 5) ? u[e] : (p == 1 || p == 4 ? v[e] : w[e]);
-        const Cx<R> b = (p == 0) ? u[e] : ((p == 1 || p == 3) ? v[e] : w[e]);
-        z[e] = Cx<R>{a.x * b.x * factor, a.y * b.y * factor};
-      }
+      if constexpr (MODE == 1) z[e] = (p == 0 ? u[e] : (p == 1 ? v[e] : w[e])) * factor;
+      else if constexpr (MODE == 3) z[e] = combined_product<R>(p, u[e], v[e], w[e], factor);
+      else z[e] = plain_product<R>(p, u[e], v[e], w[e], factor);
     }
     xl_fft<R, M, -1, 0, 1>(z, L, t, act, twl);
     // R2C post-processing needs Z(k) and Z(M - k), Z(M) = Z(0) (for M = 2^a
