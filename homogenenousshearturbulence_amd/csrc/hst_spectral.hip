@@ -59,7 +59,7 @@ __device__ __forceinline__ Cx<PR> ldp(const typename PTraits<PR>::T2 *p) {
 // 1, 2: add the products of group 1 or 2 to rhs, oldrhs as buildrhs(ODE, g);
 // 4: prepare and the five combined products of the x pass's MODE 3
 // (vv - uu, vv - ww, uv, vw, uw), the same sums regrouped.
-constexpr int RHS_ROWS = 64;
+constexpr int RHS_ROWS = 16;  // the most rows of a chunk
 template <typename PR, int MODE, bool SHIFT>
 __global__ void __launch_bounds__(256)
     k_buildrhs(Dims D, RhsArgs a, const double2 *__restrict__ V1, const double2 *__restrict__ V2,
@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(256)
   constexpr int Q0 = (MODE == 2 ? 3 : 0), Q1 = (MODE == 1 ? 3 : (FIVE ? 5 : 6));
   const int iy0 = blockIdx.y * rch, iy1 = min(iy0 + rch, D.ny);
   // FP32 products: the stencil rows of the block's chunk from LDS (read as
-  // scalar loads, each row's waited for in turn; 2.5 % faster).  FP64 keeps
+  // scalar loads, each row's waited for in turn; 2.5 % faster in chunks of 64).  FP64 keeps
   // the scalar loads: read from LDS the uniform values take VGPRs (218 -> 254)
   // and it ran 2 % slower.
   constexpr bool LROWS = sizeof(PR) == 4;
@@ -275,8 +275,20 @@ __global__ void __launch_bounds__(256)
 int launch_buildrhs(const Dims &D, int mixed, const RhsArgs &a, const double2 *V1, const double2 *V2,
                     const double2 *V3, const void *const P[6], double2 *R1, double2 *R2, void *O1, void *O2,
                     const double *der, const double *y, hipStream_t s) {
-  const int rch = RHS_ROWS;  // rows per lane: the 5-row windows re-read 4 rows per chunk
-  dim3 grid((D.ncol + 255) / 256, (D.ny + rch - 1) / rch);
+  // Rows per lane.  A chunk walks its rows one after another and its five-row
+  // windows re-read four rows, so long chunks leave a small grid's time to the
+  // latency of that walk and short ones add reads (served by the L2 where the
+  // neighbouring chunk runs beside).  16 rows where they still give 16 blocks a
+  // CU, 8 down to one and a half blocks a CU, 4 and 2 below.  Against 64 rows
+  // throughout, us (FP64, mixed): 32 x 65 x 32 130, 96 -> 15.5, 13.5 (4 rows);
+  // 63 x 128 x 63 146, 108 -> 48, 35 (8); 128 x 257 x 128 508, 349 -> 377, 262
+  // (8; 16: 407, 271); 256 x 513 x 256 3057, 1970 -> 3102, 1850 (16; 8: 3086,
+  // 1903).  Running a column block's chunks side by side on one XCD, so that the
+  // shared rows meet in its L2, is 10 % slower (128 x 257 x 128: 420, 312).
+  const int gx = (D.ncol + 255) / 256;
+  auto blocks = [&](int r) { return (long long)gx * ((D.ny + r - 1) / r); };
+  const int rch = blocks(16) >= 4096 ? 16 : (blocks(8) >= 400 ? 8 : (blocks(4) >= 128 ? 4 : 2));
+  dim3 grid(gx, (D.ny + rch - 1) / rch);
   const size_t pstride = (size_t)D.NYg * D.ncol;
   // 0 prepare, 1/2 one group, 3 all, 4 all from the five combinations, 5 as 4
   // with eta and dv/dy in V1 and V3
