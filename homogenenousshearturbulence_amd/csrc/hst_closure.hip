@@ -6,7 +6,7 @@
 //   k_cxc2r      x inverse real transform to physical values (FP64)
 //   k_samples    (9 gradients, 6 stresses) per coarse grid point
 //   k_mlp_train  forward + backward of the 9-64-64-6 tanh network for 128
-//                samples per wavefront on the matrix cores (bfloat16 operands,
+//                samples per block on the matrix cores (bfloat16 operands,
 //                FP32 accumulation), per-block partial gradients
 //   k_adam       ordered reduction of the partial gradients and the Adam step
 //   k_mlp_infer  the network on samples or on the physical gradient fields
@@ -31,6 +31,7 @@
 #include <numeric>
 #include <random>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "hst_cx.h"
@@ -47,8 +48,8 @@ constexpr int NP = HST_MLP_NPARAM;
 constexpr int NPP = NP + 2;  // row of the partial-gradient buffer: the parameters, the loss
 constexpr int OW1 = 0, OB1 = 64 * 9, OW2 = OB1 + 64, OB2 = OW2 + 64 * 64, OW3 = OB2 + 64, OB3 = OW3 + 6 * 64;
 static_assert(OB3 + 6 == NP, "parameter layout");
-constexpr int SPB = 128;        // samples per training block (one wavefront)
-constexpr int SP = 40;          // LDS row stride (bf16) of the [feature][32 samples] staging
+constexpr int SPB = 128;        // samples per training block
+constexpr int SP = 72;          // LDS row stride (bf16) of the [feature][64 samples] staging
 constexpr int MAX_PART = 2048;  // partial-gradient rows: at most SPB * MAX_PART samples per launch
 
 // ================================================================== transforms
@@ -225,49 +226,81 @@ __device__ __forceinline__ f4 mfma(const bf8 &a, const bf8 &b, const f4 &c) {
 // formed from the D fragments of output tiles 2kb and 2kb+1
 __device__ __forceinline__ int kfeat(int kb, int q, int v) { return 32 * kb + (v < 4 ? 4 * q + v : 12 + 4 * q + v); }
 
-struct WLds {
+// The weights as the instruction's operands: those of the forward pass, and
+// behind them (training) the transposed ones of the backward pass.  One image
+// of them per context is kept in global memory beside the FP32 parameters, so
+// that a block copies it to LDS in whole cache lines (gathered from the
+// parameters by every block it took 5 of the training kernel's 29 us); k_pack
+// writes it for given parameters and k_adam with each update.
+struct WFwd {
   bf8 A1[4][64];     // W1[16m+i][8q+v], K padded 9 -> 32
   bf8 A2[4][2][64];  // W2[16m+i][kfeat]
   bf8 A3[2][64];     // W3[i][kfeat], rows 6..15 zero
-  bf8 B3[4][64];     // W3[4q+v][16m+i] (v < 4): W3^T against the output errors
-  bf8 B2[4][2][64];  // W2[kfeat][16m+i]: W2^T
   float b1[64], b2[64], b3[16];
 };
+struct WBwd {
+  bf8 B3[4][64];     // W3[4q+v][16m+i] (v < 4): W3^T against the output errors
+  bf8 B2[4][2][64];  // W2[kfeat][16m+i]: W2^T
+};
+struct WImage {
+  WFwd f;
+  WBwd b;
+};
 
-__device__ void stage_weights(const float *__restrict__ par, WLds &W, int l) {
-  const int i = l & 15, q = l >> 4;
-  for (int m = 0; m < 4; m++) {
-    bf8 a;
-    for (int v = 0; v < 8; v++) {
-      const int k = 8 * q + v;
-      a[v] = (__bf16)(k < 9 ? par[OW1 + (16 * m + i) * 9 + k] : 0.0f);
-    }
-    W.A1[m][l] = a;
-    bf8 b;
-    for (int v = 0; v < 8; v++) {
-      const int o = 4 * q + v;
-      b[v] = (__bf16)((v < 4 && o < 6) ? par[OW3 + o * 64 + 16 * m + i] : 0.0f);
-    }
-    W.B3[m][l] = b;
-    for (int kb = 0; kb < 2; kb++) {
-      bf8 x, y;
-      for (int v = 0; v < 8; v++) {
-        const int f = kfeat(kb, q, v);
-        x[v] = (__bf16)par[OW2 + (16 * m + i) * 64 + f];
-        y[v] = (__bf16)par[OW2 + f * 64 + 16 * m + i];
-      }
-      W.A2[m][kb][l] = x;
-      W.B2[m][kb][l] = y;
-    }
+// parameter p (of value x) into its places of the image
+__device__ __forceinline__ void pack_param(int p, float x, WImage &w) {
+  const __bf16 h = (__bf16)x;
+  // K block, lane group and slot of feature f (the inverse of kfeat)
+  auto slot = [](int f, int &kb, int &q, int &v) {
+    const int g = f & 31;
+    kb = f >> 5;
+    q = (g & 15) >> 2;
+    v = (g & 3) + (g < 16 ? 0 : 4);
+  };
+  int kb, q, v;
+  if (p < OB1) {
+    const int r = p / 9, k = p - r * 9;
+    w.f.A1[r >> 4][(r & 15) + 16 * (k >> 3)][k & 7] = h;
+  } else if (p < OW2) {
+    w.f.b1[p - OB1] = x;
+  } else if (p < OB2) {
+    const int r = (p - OW2) >> 6, f = (p - OW2) & 63;
+    slot(f, kb, q, v);
+    w.f.A2[r >> 4][kb][(r & 15) + 16 * q][v] = h;
+    slot(r, kb, q, v);
+    w.b.B2[f >> 4][kb][(f & 15) + 16 * q][v] = h;
+  } else if (p < OW3) {
+    w.f.b2[p - OB2] = x;
+  } else if (p < OB3) {
+    const int o = (p - OW3) >> 6, f = (p - OW3) & 63;
+    slot(f, kb, q, v);
+    w.f.A3[kb][o + 16 * q][v] = h;
+    w.b.B3[f >> 4][(f & 15) + 16 * (o >> 2)][o & 3] = h;
+  } else {
+    w.f.b3[p - OB3] = x;
   }
-  for (int kb = 0; kb < 2; kb++) {
-    bf8 a;
-    for (int v = 0; v < 8; v++) a[v] = (__bf16)(i < 6 ? par[OW3 + i * 64 + kfeat(kb, q, v)] : 0.0f);
-    W.A3[kb][l] = a;
-  }
-  W.b1[l] = par[OB1 + l];
-  W.b2[l] = par[OB2 + l];
-  if (l < 16) W.b3[l] = l < 6 ? par[OB3 + l] : 0.0f;
+}
+
+// The image of the parameters; one block: the padding zero, then the entries.
+__global__ void __launch_bounds__(1024) k_pack(const float *__restrict__ par, WImage *__restrict__ img) {
+  for (int k = threadIdx.x; k < (int)(sizeof(WImage) / 4); k += 1024) ((float *)img)[k] = 0.0f;
+  __syncthreads();
+  for (int p = threadIdx.x; p < NP; p += 1024) pack_param(p, par[p], *img);
+}
+
+// a part of the image to LDS by the NT threads of a block, every load before the first store
+template <int NT, class T>
+__device__ __forceinline__ void stage_weights(const T &g, T &lds) {
+  typedef __attribute__((__vector_size__(16))) float v4;
+  constexpr int N = sizeof(T) / 16, PER = (N + NT - 1) / NT;
+  static_assert(sizeof(T) % 16 == 0, "whole vectors");
+  const v4 *src = (const v4 *)&g;
+  v4 t[PER];
+#pragma unroll
+  for (int u = 0; u < PER; u++) t[u] = src[min(u * NT + (int)threadIdx.x, N - 1)];
+#pragma unroll
+  for (int u = 0; u < PER; u++)
+    if (u * NT + (int)threadIdx.x < N) ((v4 *)&lds)[u * NT + threadIdx.x] = t[u];
 }
 
 // B operands of the next layer from the D fragments of four 16-row tiles
@@ -281,46 +314,72 @@ __device__ __forceinline__ void to_operands(const f4 h[4], bf8 B[2]) {
     }
 }
 
+// tanh x without a branch: below one, x - x^3 (45045 + 2772 x^2 + 27 x^4) / D,
+// D = 135135 + 62370 x^2 + 3150 x^4 + 28 x^6 (the seventh convergent of Lambert's
+// continued fraction, 7e-11 off at one, written as a correction to x); above,
+// +-1 -+ 2 / (exp(2 |x|) + 1), |x| cut at 10 where the correction is 4e-9.  One
+// reciprocal serves both, and since the correction is at most a quarter of the
+// result its rounding hardly shows: over 4 M arguments of 1e-8 .. 12 the largest
+// error against 64 bits is 1.33 units of the last place and the rms 0.238
+// (tanhf: 1.35 and 0.240).  A wavefront evaluates 32 a tile, most of the
+// network's instructions: k_mlp_infer 116 -> 90 us on 798,720 points.
+__device__ __forceinline__ float tanh_f(float x) {
+  const float a = fabsf(x), c = a > 10.0f ? 10.0f : a, x2 = x * x;
+  const bool small = a < 1.0f;
+  const float e = __builtin_amdgcn_exp2f(c * 2.88539008f);  // 2 / ln 2
+  const float p = -x * x2 * fmaf(x2, fmaf(x2, 27.0f, 2772.0f), 45045.0f);
+  const float q = fmaf(x2, fmaf(x2, fmaf(x2, 28.0f, 3150.0f), 62370.0f), 135135.0f);
+  const float num = small ? p : copysignf(2.0f, -x), den = small ? q : e + 1.0f;
+  return fmaf(num, __builtin_amdgcn_rcpf(den), small ? x : copysignf(1.0f, x));
+}
+
 // Forward pass of one 16-sample tile: x the input operand; h1, h2 the hidden
 // activations (FP32 D fragments), y the outputs (rows 4q+v, valid below 6).
-__device__ __forceinline__ void forward(const WLds &W, int l, const bf8 &x, f4 h1[4], f4 h2[4], f4 &y) {
+// The biases start the accumulators.
+__device__ __forceinline__ void forward(const WFwd &W, int l, const bf8 &x, f4 h1[4], f4 h2[4], f4 &y) {
   const int q = l >> 4;
-  const f4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int m = 0; m < 4; m++) {
-    const f4 z = mfma(W.A1[m][l], x, zero);
+    const f4 z = mfma(W.A1[m][l], x, *(const f4 *)(W.b1 + 16 * m + 4 * q));
 #pragma unroll
-    for (int v = 0; v < 4; v++) h1[m][v] = tanhf(z[v] + W.b1[16 * m + 4 * q + v]);
+    for (int v = 0; v < 4; v++) h1[m][v] = tanh_f(z[v]);
   }
   bf8 B[2];
   to_operands(h1, B);
 #pragma unroll
   for (int m = 0; m < 4; m++) {
-    f4 z = mfma(W.A2[m][0][l], B[0], zero);
+    f4 z = mfma(W.A2[m][0][l], B[0], *(const f4 *)(W.b2 + 16 * m + 4 * q));
     z = mfma(W.A2[m][1][l], B[1], z);
 #pragma unroll
-    for (int v = 0; v < 4; v++) h2[m][v] = tanhf(z[v] + W.b2[16 * m + 4 * q + v]);
+    for (int v = 0; v < 4; v++) h2[m][v] = tanh_f(z[v]);
   }
   to_operands(h2, B);
-  y = mfma(W.A3[0][l], B[0], zero);
+  y = mfma(W.A3[0][l], B[0], *(const f4 *)(W.b3 + 4 * q));
   y = mfma(W.A3[1][l], B[1], y);
-#pragma unroll
-  for (int v = 0; v < 4; v++) y[v] += W.b3[4 * q + v];
 }
 
-// the input operand of the sample of lane l: x[0..7] in group 0, x[8] in group 1
-template <class LoadX>
-__device__ __forceinline__ bf8 input_operand(int q, bool valid, const Norm &nm, LoadX ld) {
-  bf8 x;
+// The standardisation of a lane's inputs: features 8q .. 8q+7 in lane group q,
+// the ninth for those past it (whose operand entries are zero).
+struct LaneNorm {
+  float m[8], r[8];
+  __device__ __forceinline__ LaneNorm(const Norm &nm, int q) {
 #pragma unroll
-  for (int v = 0; v < 8; v++) {
-    const int k = 8 * q + v;
-    float xv = 0.0f;
-    if (valid && k < 9) xv = (ld(k) - nm.mx[k]) * nm.rx[k];
-    x[v] = (__bf16)xv;
+    for (int v = 0; v < 8; v++) {
+      const int k = min(8 * q + v, 8);
+      m[v] = nm.mx[k];
+      r[v] = nm.rx[k];
+    }
   }
-  return x;
-}
+  // the input operand of the sample whose features raw holds
+  template <typename In>
+  __device__ __forceinline__ bf8 operand(int q, bool valid, const In (&raw)[8]) const {
+    bf8 x;
+#pragma unroll
+    for (int v = 0; v < 8; v++)
+      x[v] = (__bf16)((valid && 8 * q + v < 9) ? ((float)raw[v] - m[v]) * r[v] : 0.0f);
+    return x;
+  }
+};
 
 struct TrainArgs {
   const float *X, *Y;
@@ -333,57 +392,90 @@ struct TrainArgs {
 // GRAD: forward, backward and the per-block partial gradients (part[blk][NPP],
 // the last two entries the sum of squared errors); otherwise the sum of
 // squared errors alone into lossp[blk].
+//
+// A block of four wavefronts takes SPB samples in passes of 64.  In a pass every
+// wavefront runs forward and backward of a 16-sample tile of its own and stages
+// activations and errors [feature][sample]; then it forms the 16 rows of the
+// weight gradients that are its own over all 64 samples, so no gradient is
+// summed across wavefronts and a wavefront holds a quarter of them.  The kernel
+// is bound by the latency of this chain (tanh, LDS, barriers) and not by the
+// matrix cores: a batch of 65,536 on one wavefront per 128 samples left half of
+// the SIMDs without work, 65 -> 32 us (25.5 with
+// tanh_f and the operand image).
+constexpr int TNT = 256, TPS = 64;  // threads; samples per pass
+static_assert(SPB % TPS == 0 && TPS == TNT / 4, "a tile of 16 samples per wavefront and pass");
+
 template <bool GRAD>
-__global__ void __launch_bounds__(64)
-    k_mlp_train(const float *__restrict__ par, Norm nm, TrainArgs ta, float *__restrict__ part,
+__global__ void __launch_bounds__(TNT)
+    k_mlp_train(const WImage *__restrict__ img, Norm nm, TrainArgs ta, float *__restrict__ part,
                 double *__restrict__ lossp) {
-  __shared__ WLds W;
-  __shared__ __attribute__((aligned(16))) __bf16 Xs[16][SP], H1s[64][SP], H2s[64][SP], DYs[16][SP], DZ2s[64][SP],
-      DZ1s[64][SP];
-  const int l = threadIdx.x, j = l & 15, q = l >> 4;
-  stage_weights(par, W, l);
-  for (int r = 9; r < 16; r++)
-    if (l < SP) Xs[r][l] = (__bf16)0.0f;
+  constexpr int NPASS = SPB / TPS, ROWS = GRAD ? 1 : 0;  // (the arrays of the backward pass are its own)
+  __shared__ WFwd W;
+  __shared__ WBwd WB[1];
+  __shared__ __attribute__((aligned(16))) __bf16 Xs[ROWS * 16 + 1][SP], H1s[ROWS * 64 + 1][SP],
+      H2s[ROWS * 64 + 1][SP], DYs[ROWS * 16 + 1][SP], DZ2s[ROWS * 64 + 1][SP], DZ1s[ROWS * 64 + 1][SP];
+  __shared__ float red[4][2 * 64 + 8];
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6, j = l & 15, q = l >> 4;
+  // the samples of every pass: index, inputs and targets, in flight while the weights are staged
+  bool valid[NPASS];
+  float xr[NPASS][8], yr[NPASS][4];
+#pragma unroll
+  for (int p = 0; p < NPASS; p++) {
+    const int64_t b = (int64_t)blockIdx.x * SPB + p * TPS + w * 16 + j;
+    valid[p] = b < ta.n;
+    const int64_t idx = (ta.mul * (ta.base + (valid[p] ? b : 0)) + ta.add) % ta.mod;
+#pragma unroll
+    for (int v = 0; v < 8; v++) xr[p][v] = ta.X[idx * 9 + min(8 * q + v, 8)];
+#pragma unroll
+    for (int v = 0; v < 4; v++) yr[p][v] = ta.Y[idx * 6 + min(4 * q + v, 5)];
+  }
+  const LaneNorm ln(nm, q);
+  float my[4], ry[4];
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    my[v] = nm.my[min(4 * q + v, 5)];
+    ry[v] = nm.ry[min(4 * q + v, 5)];
+  }
+  stage_weights<TNT>(img->f, W);
+  if constexpr (GRAD) {
+    stage_weights<TNT>(img->b, WB[0]);
+    for (int r = 9 + w; r < 16; r += 4)
+      if (l < TPS) Xs[r][l] = (__bf16)0.0f;
+  }
   __syncthreads();
   const f4 zero = {0.f, 0.f, 0.f, 0.f};
-  f4 gW2[4][4], gW1[4], gW3[4];
+  f4 gW2[4], gW1 = zero, gW3 = zero;
   float gb1[4][4], gb2[4][4], gb3[4];
+#pragma unroll
   for (int a = 0; a < 4; a++) {
-    gW1[a] = zero;
-    gW3[a] = zero;
-    for (int b = 0; b < 4; b++) { gW2[a][b] = zero; gb1[a][b] = 0.f; gb2[a][b] = 0.f; }
+    gW2[a] = zero;
     gb3[a] = 0.f;
+#pragma unroll
+    for (int v = 0; v < 4; v++) { gb1[a][v] = 0.f; gb2[a][v] = 0.f; }
   }
   float lsum = 0.0f;
-  for (int kb = 0; kb < SPB / 32; kb++) {
-#pragma unroll 1
-    for (int jt = 0; jt < 2; jt++) {
-      const int64_t b = (int64_t)blockIdx.x * SPB + kb * 32 + jt * 16 + j;
-      const bool valid = b < ta.n;
-      int64_t idx = 0;
-      if (valid) idx = (ta.mul * (ta.base + b) + ta.add) % ta.mod;
-      const bf8 x = input_operand(q, valid, nm, [&](int k) { return ta.X[idx * 9 + k]; });
-      f4 h1[4], h2[4], y;
-      forward(W, l, x, h1, h2, y);
-      f4 dy = zero;
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int o = 4 * q + v;
-        if (valid && o < 6) {
-          const float yh = (ta.Y[idx * 6 + o] - nm.my[o]) * nm.ry[o];
-          const float e = y[v] - yh;
-          lsum += e * e;
-          dy[v] = ta.scale * e;
-        }
+  for (int p = 0; p < NPASS; p++) {
+    const bf8 x = ln.operand(q, valid[p], xr[p]);
+    f4 h1[4], h2[4], y;
+    forward(W, l, x, h1, h2, y);
+    f4 dy = zero;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      if (valid[p] && 4 * q + v < 6) {
+        const float e = y[v] - (yr[p][v] - my[v]) * ry[v];
+        lsum += e * e;
+        dy[v] = ta.scale * e;
       }
-      if constexpr (!GRAD) continue;
+    }
+    if constexpr (GRAD) {
       bf8 Bd;
 #pragma unroll
       for (int v = 0; v < 4; v++) { Bd[v] = (__bf16)dy[v]; Bd[4 + v] = (__bf16)0.0f; }
       f4 dz2[4], dz1[4];
 #pragma unroll
       for (int m = 0; m < 4; m++) {
-        const f4 a = mfma(W.B3[m][l], Bd, zero);
+        const f4 a = mfma(WB[0].B3[m][l], Bd, zero);
 #pragma unroll
         for (int v = 0; v < 4; v++) dz2[m][v] = a[v] * (1.0f - h2[m][v] * h2[m][v]);
       }
@@ -391,13 +483,13 @@ __global__ void __launch_bounds__(64)
       to_operands(dz2, Bz);
 #pragma unroll
       for (int m = 0; m < 4; m++) {
-        f4 a = mfma(W.B2[m][0][l], Bz[0], zero);
-        a = mfma(W.B2[m][1][l], Bz[1], a);
+        f4 a = mfma(WB[0].B2[m][0][l], Bz[0], zero);
+        a = mfma(WB[0].B2[m][1][l], Bz[1], a);
 #pragma unroll
         for (int v = 0; v < 4; v++) dz1[m][v] = a[v] * (1.0f - h1[m][v] * h1[m][v]);
       }
       // stage [feature][sample] for the weight gradients; bias gradients in FP32
-      const int col = jt * 16 + j;
+      const int col = w * 16 + j;
 #pragma unroll
       for (int v = 0; v < 8; v++)
         if (8 * q + v < 9) Xs[8 * q + v][col] = x[v];
@@ -418,40 +510,39 @@ __global__ void __launch_bounds__(64)
         DYs[4 * q + v][col] = Bd[v];
         gb3[v] += dy[v];
       }
-    }
-    if constexpr (GRAD) {
       __syncthreads();
-      // K = the 32 samples of this block step: A rows from one array, B columns from another
-      auto rd = [&](const __bf16 *row) { return *(const bf8 *)(row + 8 * q); };
+      // K = 32 samples at a time: the wavefront's A rows from one array, B columns from another
 #pragma unroll
-      for (int mn = 0; mn < 4; mn++) {
-        const bf8 dz2r = rd(DZ2s[16 * mn + j]);
+      for (int k = 0; k < TPS / 32; k++) {
+        auto rd = [&](const __bf16 *row) { return *(const bf8 *)(row + 32 * k + 8 * q); };
+        const bf8 dz2r = rd(DZ2s[16 * w + j]);
 #pragma unroll
-        for (int mk = 0; mk < 4; mk++) gW2[mn][mk] = mfma(dz2r, rd(H1s[16 * mk + j]), gW2[mn][mk]);
-        gW1[mn] = mfma(rd(DZ1s[16 * mn + j]), rd(Xs[j]), gW1[mn]);
-        gW3[mn] = mfma(rd(DYs[j]), rd(H2s[16 * mn + j]), gW3[mn]);
+        for (int mk = 0; mk < 4; mk++) gW2[mk] = mfma(dz2r, rd(H1s[16 * mk + j]), gW2[mk]);
+        gW1 = mfma(rd(DZ1s[16 * w + j]), rd(Xs[j]), gW1);
+        gW3 = mfma(rd(DYs[j]), rd(H2s[16 * w + j]), gW3);
       }
-      __syncthreads();
+      if (p + 1 < NPASS) __syncthreads();
     }
   }
-  // sum of squared errors over the wavefront
+  // sums over the wavefront, then over the four wavefronts in order
   for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
+  if (l == 0) red[w][134] = lsum;
   if constexpr (!GRAD) {
-    if (l == 0) lossp[blockIdx.x] = (double)lsum;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      lossp[blockIdx.x] = (double)red[0][134] + (double)red[1][134] + (double)red[2][134] + (double)red[3][134];
     return;
   }
   float *pr = part + (size_t)blockIdx.x * NPP;
 #pragma unroll
-  for (int mn = 0; mn < 4; mn++)
+  for (int v = 0; v < 4; v++) {
+    const int r = 16 * w + 4 * q + v;
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int r = 16 * mn + 4 * q + v;
-#pragma unroll
-      for (int mk = 0; mk < 4; mk++) pr[OW2 + r * 64 + 16 * mk + j] = gW2[mn][mk][v];
-      if (j < 9) pr[OW1 + r * 9 + j] = gW1[mn][v];
-      if (4 * q + v < 6) pr[OW3 + (4 * q + v) * 64 + 16 * mn + j] = gW3[mn][v];
-    }
-  // bias gradients: sum over the 16 sample columns
+    for (int mk = 0; mk < 4; mk++) pr[OW2 + r * 64 + 16 * mk + j] = gW2[mk][v];
+    if (j < 9) pr[OW1 + r * 9 + j] = gW1[v];
+    if (4 * q + v < 6) pr[OW3 + (4 * q + v) * 64 + 16 * w + j] = gW3[v];
+  }
+  // bias gradients: the 16 sample columns of the wavefront, then the wavefronts
 #pragma unroll
   for (int m = 0; m < 4; m++)
 #pragma unroll
@@ -468,14 +559,19 @@ __global__ void __launch_bounds__(64)
     for (int m = 0; m < 4; m++)
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        pr[OB1 + 16 * m + 4 * q + v] = gb1[m][v];
-        pr[OB2 + 16 * m + 4 * q + v] = gb2[m][v];
+        red[w][16 * m + 4 * q + v] = gb1[m][v];
+        red[w][64 + 16 * m + 4 * q + v] = gb2[m][v];
       }
 #pragma unroll
     for (int v = 0; v < 4; v++)
-      if (4 * q + v < 6) pr[OB3 + 4 * q + v] = gb3[v];
+      if (4 * q + v < 6) red[w][128 + 4 * q + v] = gb3[v];
   }
-  if (l == 0) pr[NP] = lsum;
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t < 135) {
+    const float g = red[0][t] + red[1][t] + red[2][t] + red[3][t];
+    pr[t < 64 ? OB1 + t : (t < 128 ? OB2 + t - 64 : (t < 134 ? OB3 + t - 128 : NP))] = g;
+  }
 }
 
 // Ordered sum of nblk partial rows per parameter, then (update) the Adam step
@@ -486,7 +582,8 @@ __global__ void __launch_bounds__(64)
 constexpr int AR = 8;
 __global__ void __launch_bounds__(64 * AR)
     k_adam(float *__restrict__ par, float *__restrict__ m1, float *__restrict__ m2, const float *__restrict__ part,
-           int nblk, int update, float lr, float c1, float c2, float *__restrict__ grad, double *__restrict__ sse) {
+           int nblk, int update, float lr, float c1, float c2, float *__restrict__ grad, double *__restrict__ sse,
+           WImage *__restrict__ img) {
   __shared__ double red[AR][64];
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int p = blockIdx.x * 64 + l;
@@ -512,7 +609,9 @@ __global__ void __launch_bounds__(64 * AR)
   const float a = 0.9f * m1[p] + 0.1f * gf, s = 0.999f * m2[p] + 0.001f * gf * gf;
   m1[p] = a;
   m2[p] = s;
-  par[p] -= lr * (a * c1) / (sqrtf(s * c2) + 1e-8f);
+  const float x = par[p] - lr * (a * c1) / (sqrtf(s * c2) + 1e-8f);
+  par[p] = x;
+  pack_param(p, x, *img);
 }
 
 struct InferIO {
@@ -525,31 +624,68 @@ struct InferIO {
   int mode;
 };
 
-constexpr int INFER_TILES = 32;  // 16-sample tiles per block: the weight staging is paid once per 512 samples
+// One 16-sample tile per wavefront at a time, the next tile's inputs loaded
+// while this one is computed.  The weights stay in registers, which leaves two
+// wavefronts a SIMD: two blocks of four a CU (three blocks, without: 5 % slower).
+// The vector ALU bounds it (about 900 instructions a tile, two thirds of them
+// tanh): 798,720 points take 82 us against 405 with one wavefront a block, 32
+// tiles each, tanhf and the weights gathered by every block.
+constexpr int INFER_NT = 256, INFER_BLOCKS = 256 * 2;
 
-__global__ void __launch_bounds__(64) k_mlp_infer(const float *__restrict__ par, Norm nm, InferIO io) {
-  __shared__ WLds W;
-  const int l = threadIdx.x, j = l & 15, q = l >> 4;
-  stage_weights(par, W, l);
+template <int MODE>
+__global__ void __launch_bounds__(INFER_NT) k_mlp_infer(const WImage *__restrict__ img, Norm nm, InferIO io) {
+  __shared__ WFwd W;
+  const int l = threadIdx.x & 63, j = l & 15, q = l >> 4;
+  stage_weights<INFER_NT>(img->f, W);
   __syncthreads();
-  for (int jt = 0; jt < INFER_TILES; jt++) {
-    const int64_t s = ((int64_t)blockIdx.x * INFER_TILES + jt) * 16 + j;
+  const int64_t ntile = (io.n + 15) / 16, step = (int64_t)gridDim.x * (INFER_NT / 64);
+  typedef typename std::conditional<MODE == 0, float, double>::type In;
+  const LaneNorm ln(nm, q);
+  float my[4], sy[4];
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    my[v] = nm.my[min(4 * q + v, 5)];
+    sy[v] = nm.sy[min(4 * q + v, 5)];
+  }
+  // a tile's inputs, without a branch (past the last feature or sample: the last again)
+  auto fetch = [&](int64_t tile, In (&raw)[8]) {
+    const int64_t s = min(tile * 16 + j, io.n - 1);
+#pragma unroll
+    for (int v = 0; v < 8; v++) {
+      const int k = min(8 * q + v, 8);
+      if constexpr (MODE == 0) raw[v] = io.X[s * 9 + k];
+      else raw[v] = io.gin[(size_t)k * io.fs + s];
+    }
+  };
+  int64_t tile = (int64_t)blockIdx.x * (INFER_NT / 64) + (threadIdx.x >> 6);
+  if (tile >= ntile) return;
+  In cur[8], nxt[8];
+  fetch(tile, cur);
+  for (; tile < ntile; tile += step) {
+    fetch(min(tile + step, ntile - 1), nxt);
+    const int64_t s = tile * 16 + j;
     const bool valid = s < io.n;
-    bf8 x;
-    if (io.mode == 0) x = input_operand(q, valid, nm, [&](int k) { return io.X[s * 9 + k]; });
-    else x = input_operand(q, valid, nm, [&](int k) { return (float)io.gin[(size_t)k * io.fs + s]; });
+    const bf8 x = ln.operand(q, valid, cur);
     f4 h1[4], h2[4], y;
     forward(W, l, x, h1, h2, y);
-    if (!valid) continue;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       const int o = 4 * q + v;
-      if (o >= 6) continue;
-      const float t = y[v] * nm.sy[o] + nm.my[o];
-      if (io.mode == 0) io.Y[s * 6 + o] = t;
+      if (!valid || o >= 6) continue;
+      const float t = y[v] * sy[v] + my[v];
+      if constexpr (MODE == 0) io.Y[s * 6 + o] = t;
       else io.tout[(size_t)o * io.fs + s] = (double)t;
     }
+#pragma unroll
+    for (int v = 0; v < 8; v++) cur[v] = nxt[v];
   }
+}
+
+static void run_infer(const WImage *img, const Norm &nm, const InferIO &io, hipStream_t st) {
+  const int64_t tiles = (io.n + 15) / 16, per = INFER_NT / 64;
+  dim3 grid((unsigned)std::min<int64_t>((tiles + per - 1) / per, INFER_BLOCKS));
+  if (io.mode == 0) hipLaunchKernelGGL(k_mlp_infer<0>, grid, dim3(INFER_NT), 0, st, img, nm, io);
+  else hipLaunchKernelGGL(k_mlp_infer<1>, grid, dim3(INFER_NT), 0, st, img, nm, io);
 }
 
 // sums (pass 0) or sums of squared deviations (pass 1) of the 15 columns, per block
@@ -640,6 +776,7 @@ struct hst_closure {
   int fine_ny = 0;
   int64_t cap = 0, count = 0;
   float *X = nullptr, *Yd = nullptr;
+  WImage *img = nullptr;  // the parameters as the matrix cores' operands
   float *par = nullptr, *m1 = nullptr, *m2 = nullptr, *part = nullptr, *gradd = nullptr;
   double *sse = nullptr, *lossp = nullptr, *mom = nullptr, *meand = nullptr;
   int64_t adam_t = 0;
@@ -757,8 +894,7 @@ int stress(hst_closure *c, const double2 *const U[3], double sx, double sz, hipS
   io.fs = c->fs();
   io.n = (int64_t)c->fs();
   io.mode = 1;
-  hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)((io.n + 16 * INFER_TILES - 1) / (16 * INFER_TILES))), dim3(64), 0,
-                     st, c->par, make_norm(c->norm), io);
+  run_infer(c->img, make_norm(c->norm), io, st);
   Cx<double> *Hp = c->Hc;  // the z-inverse output is free again
   switch (D.nxd) {
 #define XC(n) case n: run_cxr2c<n>(D, c->phys + 9 * c->fs(), Hp, c->twx, c->twh, st); break;
@@ -812,7 +948,7 @@ void release(hst_closure *c) {
   if (c->own) (void)hipStreamSynchronize(c->own);
   void *ptrs[] = {c->d_der, c->d_dyl, c->d_f0, c->twz, c->twx, c->twh, c->fields, c->Gy, c->XR, c->Hc, c->phys,
                   c->stage, c->d_j0, c->d_w, c->X, c->Yd, c->par, c->m1, c->m2, c->part, c->gradd, c->sse,
-                  c->lossp, c->mom, c->meand};
+                  c->lossp, c->mom, c->meand, c->img};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (c->tables) free_fft_tables(c->tables);
@@ -898,6 +1034,7 @@ int hst_closure_create(const hst_deck *coarse, int64_t capacity, hst_closure **o
     MAL(c->X, (size_t)capacity * 9 * sizeof(float));
     MAL(c->Yd, (size_t)capacity * 6 * sizeof(float));
   }
+  MAL(c->img, sizeof(WImage));
   MAL(c->par, NP * sizeof(float));
   MAL(c->m1, NP * sizeof(float));
   MAL(c->m2, NP * sizeof(float));
@@ -1120,6 +1257,9 @@ int hst_closure_set_params(hst_closure *c, const float *params) {
   CHK(hipMemcpy(c->par, params, NP * sizeof(float), hipMemcpyHostToDevice));
   CHK(hipMemset(c->m1, 0, NP * sizeof(float)));
   CHK(hipMemset(c->m2, 0, NP * sizeof(float)));
+  hipLaunchKernelGGL(k_pack, dim3(1), dim3(1024), 0, c->own, c->par, c->img);
+  CHK(hipGetLastError());
+  CHK(hipStreamSynchronize(c->own));  // the image is read on the live state's stream too
   c->adam_t = 0;
   c->have_params = true;
   return 0;
@@ -1139,10 +1279,10 @@ int hst_closure_grad(hst_closure *c, int64_t first, int64_t n, float *grad, doub
   hipStream_t st = c->own;
   TrainArgs ta{c->X, c->Yd, n, first, 1, 0, INT64_MAX, (float)(2.0 / ((double)n * 6.0))};
   const int nblk = (int)((n + SPB - 1) / SPB);
-  hipLaunchKernelGGL(k_mlp_train<true>, dim3(nblk), dim3(64), 0, st, c->par, make_norm(c->norm), ta, c->part,
+  hipLaunchKernelGGL(k_mlp_train<true>, dim3(nblk), dim3(TNT), 0, st, c->img, make_norm(c->norm), ta, c->part,
                      c->lossp);
   hipLaunchKernelGGL(k_adam, dim3((NP + 1 + 63) / 64), dim3(64 * AR), 0, st, c->par, c->m1, c->m2, c->part, nblk, 0,
-                     0.0f, 0.0f, 0.0f, c->gradd, c->sse);
+                     0.0f, 0.0f, 0.0f, c->gradd, c->sse, c->img);
   CHK(hipGetLastError());
   double sse = 0.0;
   if (grad) CHK(hipMemcpyAsync(grad, c->gradd, NP * sizeof(float), hipMemcpyDeviceToHost, st));
@@ -1162,7 +1302,7 @@ static int eval_loss(hst_closure *c, int64_t first, int64_t n, double *loss) {
     const int64_t m = std::min(chunk, n - b0);
     TrainArgs ta{c->X, c->Yd, m, first + b0, 1, 0, INT64_MAX, 0.0f};
     const int nblk = (int)((m + SPB - 1) / SPB);
-    hipLaunchKernelGGL(k_mlp_train<false>, dim3(nblk), dim3(64), 0, st, c->par, make_norm(c->norm), ta, c->part,
+    hipLaunchKernelGGL(k_mlp_train<false>, dim3(nblk), dim3(TNT), 0, st, c->img, make_norm(c->norm), ta, c->part,
                        c->lossp);
     CHK(hipGetLastError());
     CHK(hipMemcpyAsync(h.data(), c->lossp, nblk * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -1201,9 +1341,9 @@ int hst_closure_train(hst_closure *c, int epochs, int batch, double lr, uint64_t
       const double t = (double)c->adam_t;
       const float c1 = (float)(1.0 / (1.0 - std::pow(0.9, t))), c2 = (float)(1.0 / (1.0 - std::pow(0.999, t)));
       TrainArgs ta{c->X, c->Yd, batch, b * batch, mul, add, n_train, (float)(2.0 / ((double)batch * 6.0))};
-      hipLaunchKernelGGL(k_mlp_train<true>, dim3(nblk), dim3(64), 0, st, c->par, nm, ta, c->part, c->lossp);
+      hipLaunchKernelGGL(k_mlp_train<true>, dim3(nblk), dim3(TNT), 0, st, c->img, nm, ta, c->part, c->lossp);
       hipLaunchKernelGGL(k_adam, dim3((NP + 1 + 63) / 64), dim3(64 * AR), 0, st, c->par, c->m1, c->m2, c->part, nblk,
-                         1, (float)lr, c1, c2, c->gradd, dsse + b);
+                         1, (float)lr, c1, c2, c->gradd, dsse + b, c->img);
     }
     hipError_t err = hipGetLastError();
     if (err == hipSuccess) err = hipMemcpyAsync(h.data(), dsse, sizeof(double) * nb, hipMemcpyDeviceToHost, st);
@@ -1244,8 +1384,7 @@ int hst_closure_predict(hst_closure *c, int64_t n, const float *x, float *y) {
   InferIO io{dx, dy, nullptr, nullptr, 0, n, 0};
   hipError_t e = hipMemcpyAsync(dx, x, (size_t)n * 9 * sizeof(float), hipMemcpyHostToDevice, st);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)((n + 16 * INFER_TILES - 1) / (16 * INFER_TILES))), dim3(64), 0,
-                       st, c->par, make_norm(c->norm), io);
+    run_infer(c->img, make_norm(c->norm), io, st);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipMemcpyAsync(y, dy, (size_t)n * 6 * sizeof(float), hipMemcpyDeviceToHost, st);
