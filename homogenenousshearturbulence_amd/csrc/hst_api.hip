@@ -79,8 +79,9 @@ struct State {
   // solves and the next substep's transforms, and is joined before the next
   // buildrhs (or before any other entry point)
   hipStream_t side = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_tab = nullptr;
   bool side_pending = false;
+  bool tab_pending = false;  // factor tables under way on the side stream
   double2 *XRo[2] = {nullptr, nullptr};
   double2 *PX = nullptr, *PZ = nullptr;  // node phases of the exact shift
   double *exz_acc = nullptr;             // column energies summed over the outstats calls
@@ -523,35 +524,84 @@ static int ghosts(int nf, double2 *const *f, double sx, double sz) {
   return run("ghosts", nf * 8.0 * S.D.ncol * 16.0, [&] { return launch_ghosts(S.D, nf, f, sx, sz, S.stream); });
 }
 
+// Memory for the factor tables of slot k, or false (and no tables from then
+// on) when they do not fit.
+static bool penta_slot(int k) {
+  if (S.ptab[k][0]) return true;
+  const size_t tb = penta_table_bytes(S.D);
+  size_t free_b = 0, total_b = 0;
+  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < 2 * tb + ((size_t)4 << 30)) {
+    S.ptab_off = true;
+    return false;
+  }
+  if (hipMalloc(&S.ptab[k][0], tb) != hipSuccess || hipMalloc(&S.ptab[k][1], tb) != hipSuccess) {
+    (void)hipGetLastError();
+    S.ptab_off = true;
+    return false;
+  }
+  S.bytes_held += 2 * (int64_t)tb;
+  return true;
+}
+
+// the main stream waits for factor tables under way on the side stream
+static int join_tables() {
+  if (!S.tab_pending) return 0;
+  S.tab_pending = false;
+  HIPCHK(hipStreamWaitEvent(S.stream, S.ev_tab, 0));
+  return 0;
+}
+
+// The factor tables of a time step's three lambdas, in one launch, when they
+// are not those held: on the side stream beside the substep's transforms (a
+// step whose length changes, as under the CFL rule, needs new ones each time).
+static int penta_prebuild(double deltat) {
+  if (S.ptab_off) return 0;
+  double lam[3];
+  bool have = true;
+  for (int i = 0; i < 3; i++) {
+    lam[i] = RK[i][0] / deltat;
+    bool found = false;
+    for (int k = 0; k < 3; k++) found = found || (S.ptab[k][0] && S.ptab_lam[k] == lam[i]);
+    have = have && found;
+  }
+  if (have) return 0;
+  void *tabs[6];
+  for (int k = 0; k < 3; k++) {
+    if (!penta_slot(k)) return 0;
+    tabs[2 * k] = S.ptab[k][0];
+    tabs[2 * k + 1] = S.ptab[k][1];
+    S.ptab_lam[k] = 0.0;  // (no lambda, if the launch fails)
+  }
+  const bool serial = S.prof || S.serial;
+  hipStream_t st = serial ? S.stream : S.side;
+  if (!serial) {  // the solves that read the old tables come first
+    HIPCHK(hipEventRecord(S.ev_fork, S.stream));
+    HIPCHK(hipStreamWaitEvent(S.side, S.ev_fork, 0));
+  }
+  if (int rc = run_on(st, "penta_factor", 6.0 * (double)penta_table_bytes(S.D),
+                      [&] { return launch_penta_factor(S.D, 3, lam, tabs, S.d_der, st); }))
+    return rc;
+  if (!serial) {
+    HIPCHK(hipEventRecord(S.ev_tab, S.side));
+    S.tab_pending = true;
+  }
+  for (int k = 0; k < 3; k++) S.ptab_lam[k] = lam[k];
+  S.ptab_next = 0;
+  return 0;
+}
+
 // The factor tables for lambda (D2V, ETA), or null when they do not fit.
 static const void *const *penta_tables(double lambda) {
-  if (S.ptab_off) return nullptr;
+  if (S.ptab_off || join_tables()) return nullptr;
   for (int k = 0; k < 3; k++)
     if (S.ptab[k][0] && S.ptab_lam[k] == lambda) return S.ptab[k];
   const int k = S.ptab_next;
-  const size_t tb = penta_table_bytes(S.D);
-  if (!S.ptab[k][0]) {
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < 2 * tb + ((size_t)4 << 30)) {
-      S.ptab_off = true;
-      return nullptr;
-    }
-    if (hipMalloc(&S.ptab[k][0], tb) != hipSuccess || hipMalloc(&S.ptab[k][1], tb) != hipSuccess) {
-      (void)hipGetLastError();
-      S.ptab_off = true;
-      return nullptr;
-    }
-    S.bytes_held += 2 * (int64_t)tb;
-  }
-  const int kinds[2] = {HST_KIND_D2V, HST_KIND_ETA};
-  for (int j = 0; j < 2; j++) {
-    int rc = run("penta_factor", (double)tb, [&] {
-      return launch_penta_factor(S.D, kinds[j], lambda, S.d_der, S.ptab[k][j], S.stream);
-    });
-    if (rc) {
-      S.ptab_off = true;
-      return nullptr;
-    }
+  if (!penta_slot(k)) return nullptr;
+  S.ptab_lam[k] = 0.0;
+  if (run("penta_factor", 2.0 * (double)penta_table_bytes(S.D),
+          [&] { return launch_penta_factor(S.D, 1, &lambda, S.ptab[k], S.d_der, S.stream); })) {
+    S.ptab_off = true;
+    return nullptr;
   }
   S.ptab_lam[k] = lambda;
   S.ptab_next = (k + 1) % 3;
@@ -737,6 +787,7 @@ static void release() {
   if (S.side) (void)hipStreamDestroy(S.side);
   if (S.ev_fork) (void)hipEventDestroy(S.ev_fork);
   if (S.ev_join) (void)hipEventDestroy(S.ev_join);
+  if (S.ev_tab) (void)hipEventDestroy(S.ev_tab);
   for (double2 *p : S.XRo) if (p) (void)hipFree(p);
   if (S.PX) (void)hipFree(S.PX);
   if (S.exz_acc) (void)hipFree(S.exz_acc);
@@ -808,6 +859,7 @@ int hst_gpu_init(const hst_deck *deck, int precision) {
   HIPCHK(hipStreamCreate(&S.side));
   HIPCHK(hipEventCreateWithFlags(&S.ev_fork, hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&S.ev_join, hipEventDisableTiming));
+  HIPCHK(hipEventCreateWithFlags(&S.ev_tab, hipEventDisableTiming));
   if (const char *e = std::getenv("HST_SERIAL")) S.serial = std::atoi(e) != 0;
   // HST_NO_TABLES=1: no factor tables (the path taken when they do not fit in
   // device memory): the exact shift of rhs runs apart from the line solves,
@@ -1248,6 +1300,7 @@ int hst_gpu_timestep(double deltat, double *time, double *cfl) {
   const bool compact = !S.deck.linear && g_hook == nullptr && !stokes_active() && !damping_active();
   if (!compact)
     if (int rc = restore_uw()) return rc;
+  if (int rc = penta_prebuild(deltat)) return rc;
   for (int i = 0; i < 3; i++) {
     const double *ode = RK[i];
     int rc = 0;

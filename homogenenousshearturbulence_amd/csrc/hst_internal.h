@@ -40,6 +40,7 @@ struct Dims {
   // columns, so that every row starts on a 4 KB boundary (column sweeps over
   // such rows measured 7-10 % faster than over rows 16 B off the lines)
   int ncs;
+  int exact;  // the deck's exact_shift
   double alfa0, beta0, ni, S, factor, dx, dz;
 };
 
@@ -107,11 +108,14 @@ int launch_buildrhs(const Dims &D, int mixed, const RhsArgs &a, const double2 *V
 int launch_penta(const Dims &D, int nsys, const int *kinds, double lambda, const double2 *const *src,
                  double2 *const *dst, const PentaWS *ws, const void *const *tabs, const double *der, double sx,
                  double sz, hipStream_t s);
-// The matrix part of the D2V or ETA lines for lambda: per (ix, |iz|) group
-// the factorisation's state every 8 rows, from which the solves recompute
-// the rows (penta_table_bytes of device memory).
+// The matrix part of the D2V and ETA lines for each of nlam lambdas (tabs: D2V,
+// ETA of the first, of the second, ..; penta_table_bytes of device memory each):
+// per (ix, |iz|) group the whole factorisation where penta_full_tables says so,
+// else its state every 8 rows, from which the solves recompute the rows.
+bool penta_full_tables(const Dims &D);
 size_t penta_table_bytes(const Dims &D);
-int launch_penta_factor(const Dims &D, int kind, double lambda, const double *der, void *tab, hipStream_t s);
+int launch_penta_factor(const Dims &D, int nlam, const double *lambda, void *const *tabs, const double *der,
+                        hipStream_t s);
 
 // D0-type solves with the shared factorisation.  rhs_mode 0: D0 x = src;
 // 1: D0 x = D1 src (src ghost rows filled).  out_mode 0: x into dst;

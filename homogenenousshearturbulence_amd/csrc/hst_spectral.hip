@@ -422,19 +422,22 @@ __device__ __forceinline__ double coefk(double lam, double ni, double kk, const 
 // Row pipelines of the per-column recurrences: body(i, v) for i = 0..n-1
 // (ascending) or n-1..0 (descending) with v = load(i) issued PF rows ahead,
 // so that a wavefront keeps PF rows of loads in flight while its recurrence
-// runs.  n, i are uniform over the wavefront.
-template <int PF, class T, class LOAD, class BODY>
+// runs.  n, i are uniform over the wavefront.  CLAMP: the loads past the end
+// read the last row again instead of being left out, so that a group of PF rows
+// is one block without a branch (5 to 15 % faster where the rows' latency
+// counts; the fused shift and solve of the large grids spills with it).
+template <int PF, class T, bool CLAMP = true, class LOAD, class BODY>
 __device__ __forceinline__ void rows_ascending(int n, LOAD load, BODY body) {
   T buf[PF];
 #pragma unroll
   for (int k = 0; k < PF; k++)
-    if (k < n) buf[k] = load(k);
+    if (CLAMP || k < n) buf[k] = load(CLAMP ? min(k, n - 1) : k);
   int i = 0;
   for (; i + PF <= n; i += PF) {
 #pragma unroll
     for (int k = 0; k < PF; k++) {
       const T v = buf[k];
-      if (i + k + PF < n) buf[k] = load(i + k + PF);
+      if (CLAMP || i + k + PF < n) buf[k] = load(CLAMP ? min(i + k + PF, n - 1) : i + k + PF);
       body(i + k, v);
     }
   }
@@ -443,9 +446,9 @@ __device__ __forceinline__ void rows_ascending(int n, LOAD load, BODY body) {
     if (i + k < n) body(i + k, buf[k]);
 }
 
-template <int PF, class T, class LOAD, class BODY>
+template <int PF, class T, bool CLAMP = true, class LOAD, class BODY>
 __device__ __forceinline__ void rows_descending(int n, LOAD load, BODY body) {
-  rows_ascending<PF, T>(
+  rows_ascending<PF, T, CLAMP>(
       n, [&](int k) { return load(n - 1 - k); }, [&](int k, const T &v) { body(n - 1 - k, v); });
 }
 
@@ -453,7 +456,7 @@ struct PentaArgs {
   const double2 *src[2];
   double2 *dst[2];
   PentaWS ws[2];
-  const double4 *tab[2];  // factor rows per (ix, |iz|) group, or null: the workspace holds them
+  const void *tab[2];  // the factorisation per (ix, |iz|) group, or null: the workspace holds it
 };
 
 // a row of the elimination workspace, as the back substitution reads it
@@ -559,21 +562,106 @@ static int pair_lanes(const Dims &D) { return (D.NXm * (D.nz + 1) + 31) / 32 * 6
 // the chunk.  Columns (ix, iz) and (ix, -iz) share k^2 and so every bit of
 // these rows.
 constexpr int PC = 8;
-template <int K>
-__global__ void __launch_bounds__(256) k_penta_factor(Dims D, double lam, const double *__restrict__ der,
-                                                      double4 *__restrict__ tab) {
-  const int ng = (D.nx + 1) * (D.nz + 1);
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= ng) return;
+
+// The whole factorisation of every group instead, for grids whose line solves
+// are bound by the latency of a row and not by HBM (penta_full_tables): per row
+// the multipliers, the inverse pivot, the upper entries, the border columns and
+// the record's weights, so that neither sweep of a line recomputes a pivot.  A
+// group's arrays are [row][g] and the record's real entries [k][g].
+constexpr int PF_REC = 17;  // u(mi-2)1 and the 16 entries of border_solve's rr
+struct PentaFull {
+  double4 *f;  // l2, l1, 1/pivot, w
+  double4 *b;  // t1, t2, p, q
+  double *v;   // the record's second weight
+  double *rec;
+};
+__host__ __device__ inline size_t penta_full_bytes(int mi, size_t ng) {
+  return ng * ((size_t)mi * 9 + PF_REC) * sizeof(double);
+}
+__host__ __device__ inline PentaFull penta_full_view(void *tab, int mi, size_t ng) {
+  PentaFull t;
+  t.f = (double4 *)tab;
+  t.b = t.f + ng * mi;
+  t.v = (double *)(t.b + ng * mi);
+  t.rec = t.v + ng * mi;
+  return t;
+}
+
+// Copies n doubles to LDS by a block of NT threads, sixteen loads of a thread
+// in flight.
+template <int NT>
+__device__ __forceinline__ void rows_to_lds(double *lds, const double *__restrict__ g, int n) {
+  for (int b0 = 0; b0 < n; b0 += 16 * NT) {
+    double v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = g[min(b0 + u * NT + (int)threadIdx.x, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 16; u++)
+      if (b0 + u * NT + (int)threadIdx.x < n) lds[b0 + u * NT + threadIdx.x] = v[u];
+  }
+  __syncthreads();
+}
+
+struct FactorArgs {
+  double lam[3];
+  void *tab[6];  // lam 0 D2V, lam 0 ETA, lam 1 D2V, ..
+};
+
+template <int K, bool FULL>
+__device__ __forceinline__ void penta_factor_group(const Dims &D, int g, double lam, const double *__restrict__ der,
+                                                   void *__restrict__ tab) {
+  const int mi = D.ny - 2;
+  const size_t ng = (size_t)(D.nx + 1) * (D.nz + 1);
   const int ix = g / (D.nz + 1), iz = g - ix * (D.nz + 1);
   const double al = D.alfa0 * ix, be = D.beta0 * iz;
   const double kk = al * al + be * be;
   PentaFactor f;
-  for (int i = 0; i < D.ny - 2; i++) {
-    if (i % PC == 0) f.save(tab + (size_t)(2 * (i / PC)) * ng + g, tab + (size_t)(2 * (i / PC) + 1) * ng + g);
-    double l2, l1, rp, t1, t2, p, q;
-    f.step<K>(i, lam, D.ni, kk, der, l2, l1, rp, t1, t2, p, q);
+  if constexpr (FULL) {
+    const PentaFull t = penta_full_view(tab, mi, ng);
+#pragma unroll 2
+    for (int i = 0; i < mi; i++) {
+      double l2, l1, rp, t1, t2, p, q;
+      f.step<K>(i, lam, D.ni, kk, der, l2, l1, rp, t1, t2, p, q);
+      t.f[ng * i + g] = make_double4(l2, l1, rp, f.ww);
+      t.b[ng * i + g] = make_double4(t1, t2, p, q);
+      t.v[ng * i + g] = f.vv;
+    }
+    const double r[PF_REC] = {f.u21, f.sp0, f.sq0, f.w2 * f.u22 + f.w1 * f.u11, f.w1 * f.u12, f.sp1, f.sq1,
+                              f.v2 * f.u22 + f.v1 * f.u11, f.v1 * f.u12, f.p2 - f.u21 * f.p1, f.q2 - f.u21 * f.q1,
+                              f.u22 - f.u21 * f.u11, -f.u21 * f.u12, f.p1, f.q1, f.u11, f.u12};
+#pragma unroll
+    for (int k = 0; k < PF_REC; k++) t.rec[ng * k + g] = r[k];
+  } else {
+    double4 *t = (double4 *)tab;
+    for (int i = 0; i < mi; i++) {
+      if (i % PC == 0) f.save(t + (size_t)(2 * (i / PC)) * ng + g, t + (size_t)(2 * (i / PC) + 1) * ng + g);
+      double l2, l1, rp, t1, t2, p, q;
+      f.step<K>(i, lam, D.ni, kk, der, l2, l1, rp, t1, t2, p, q);
+    }
   }
+}
+
+// blockIdx.y: the pair (lambda, kind).  CL: the stencil rows from a copy in LDS
+// (ny <= 409), as everywhere here because scalar loads are waited for row by row.
+template <bool FULL, int CL>
+__global__ void __launch_bounds__(64) k_penta_factor(Dims D, FactorArgs a, const double *__restrict__ derg) {
+  extern __shared__ double ders[];
+  if constexpr (CL) rows_to_lds<64>(ders, derg, D.ny * 20);
+  const double *const der = CL ? ders : derg;
+  const int g = blockIdx.x * 64 + threadIdx.x, c = blockIdx.y;
+  if (g >= (D.nx + 1) * (D.nz + 1)) return;
+  const double lam = a.lam[c >> 1];
+  if (c & 1) penta_factor_group<KETA, FULL>(D, g, lam, der, a.tab[c]);
+  else penta_factor_group<KD2V, FULL>(D, g, lam, der, a.tab[c]);
+}
+
+// The record's real entries of a group into border_solve's order; the
+// multiplier u(mi-2)1 is returned.
+__device__ __forceinline__ double penta_record(const PentaFull &t, size_t ng, int g, double (&rr)[25]) {
+  constexpr int at[PF_REC] = {0, 3, 4, 5, 6, 9, 10, 11, 12, 15, 16, 17, 18, 21, 22, 23, 24};
+#pragma unroll
+  for (int k = 1; k < PF_REC; k++) rr[at[k]] = t.rec[ng * k + g];
+  return t.rec[g];
 }
 
 // The back substitution of one line from its top row down (penta_backward,
@@ -619,6 +707,27 @@ __device__ __forceinline__ void penta_back(const Dims &D, int g, double lam, dou
       }
     }
   }
+}
+
+// The back substitution of one line from the whole factorisation; xs: the row
+// stride of XR.
+constexpr int PFB = 8;
+__device__ __forceinline__ void penta_full_back(const Dims &D, int col, int g, const PentaFull &t, C zb1, C zb2, C x1,
+                                                C x2, const double2 *__restrict__ XR, size_t xs,
+                                                double2 *__restrict__ dst) {
+  const size_t nc = D.ncol, ng = (size_t)(D.nx + 1) * (D.nz + 1);
+  struct Bwd {
+    C xr;
+    double4 b;
+  };
+  rows_descending<PFB, Bwd>(
+      D.ny - 2, [&](int i) { return Bwd{ld(XR + (size_t)i * xs + col), t.b[ng * i + g]}; },
+      [&](int i, const Bwd &r) {
+        const C x = r.xr - r.b.z * zb1 - r.b.w * zb2 - r.b.x * x1 - r.b.y * x2;
+        st(dst + (size_t)(i + 2) * nc + col, x);
+        x2 = x1;
+        x1 = x;
+      });
 }
 
 // One cyclic pentadiagonal line per lane (line_solve, src/hst_linsolve.f90:147-483,
@@ -699,6 +808,71 @@ __device__ __forceinline__ void penta_line(const Dims &D, int col, int ix, int i
   }
 }
 
+// penta_line from the whole factorisation: four real multiply-adds a component
+// and row in the two sweeps, PFF rows of the right-hand side and the factors in
+// flight (12 and 16 measure the same).  The same operations on the same numbers
+// as with the checkpoints.  Bound by the rate of one wavefront's memory requests
+// a CU: at 63 x 128 x 63, 100 B a row and column in 52 us are 4 TB/s.
+constexpr int PFF = 8;
+template <int K>
+__device__ __forceinline__ void penta_full_line(const Dims &D, int col, int ix, int iz, int g, double lam,
+                                                const double *__restrict__ der, const double2 *__restrict__ src,
+                                                double2 *__restrict__ dst, double2 *__restrict__ XR,
+                                                const PentaFull &t, double sx, double sz) {
+  const size_t nc = D.ncol, ng = (size_t)(D.nx + 1) * (D.nz + 1);
+  const int m = D.ny, mi = m - 2;
+  if (ix == 0 && iz == 0 && K == KD2V) {
+    for (int i = 0; i < m; i++) st(dst + (size_t)(i + 2) * nc + col, C{0.0, 0.0});
+    return;
+  }
+  const double al = D.alfa0 * ix, be = D.beta0 * iz;
+  const double kk = al * al + be * be, ni = D.ni;
+  struct Fwd {
+    C b;
+    double4 f;
+    double v;
+  };
+  C x1{0, 0}, x2{0, 0}, sx0{0, 0}, sx1{0, 0};
+  rows_ascending<PFF, Fwd>(
+      mi, [&](int i) { return Fwd{ld(src + (size_t)(i + 2) * nc + col), t.f[ng * i + g], t.v[ng * i + g]}; },
+      [&](int i, const Fwd &r) {
+        const C bx = (r.b - r.f.x * x2 - r.f.y * x1) * r.f.z;
+        st(XR + (size_t)i * nc + col, bx);
+        sx0 = sx0 + r.f.w * bx;
+        sx1 = sx1 + r.v * bx;
+        x2 = x1;
+        x1 = bx;
+      });
+  double rr[25];
+  const double u21 = penta_record(t, ng, g, rr);
+  const C xm2 = x2 - u21 * x1, xm1 = x1;
+  const C r25 = ld(src + (size_t)(m - 2 + 2) * nc + col), r27 = ld(src + (size_t)(m - 1 + 2) * nc + col);
+  const int ga = m - 2;
+  const C ph = cexpi(-(D.alfa0 * ix * sx + D.beta0 * iz * sz));
+  C b1, b2;
+  border_solve(rr, coefk<K>(lam, ni, kk, der, ga, -2), coefk<K>(lam, ni, kk, der, ga, -1),
+               coefk<K>(lam, ni, kk, der, ga, 0), coefk<K>(lam, ni, kk, der, ga, 1),
+               coefk<K>(lam, ni, kk, der, ga, 2), coefk<K>(lam, ni, kk, der, ga + 1, -2),
+               coefk<K>(lam, ni, kk, der, ga + 1, -1), coefk<K>(lam, ni, kk, der, ga + 1, 0),
+               coefk<K>(lam, ni, kk, der, ga + 1, 1), coefk<K>(lam, ni, kk, der, ga + 1, 2), ph, sx0, sx1, xm2,
+               xm1, r25, r27, b1, b2);
+  st(dst + (size_t)(m - 2 + 2) * nc + col, b1);
+  st(dst + (size_t)(m - 1 + 2) * nc + col, b2);
+  penta_full_back(D, col, g, t, conj(ph) * b1, conj(ph) * b2, b1, b2, XR, nc, dst);
+}
+
+__global__ void __launch_bounds__(64)
+    k_penta_full(Dims D, PentaArgs pa, double lam, const double *__restrict__ der, double sx, double sz) {
+  const int l = xcd_linear();
+  const int sys = l / gridDim.x;
+  int ix, iz, col, g;
+  if (!pair_lane(D, (l % gridDim.x) * 64 + threadIdx.x, ix, iz, col, g)) return;
+  const size_t ng = (size_t)(D.nx + 1) * (D.nz + 1);
+  const PentaFull t = penta_full_view((void *)pa.tab[sys], D.ny - 2, ng);
+  if (sys == 0) penta_full_line<KD2V>(D, col, ix, iz, g, lam, der, pa.src[0], pa.dst[0], pa.ws[0].XR, t, sx, sz);
+  else penta_full_line<KETA>(D, col, ix, iz, g, lam, der, pa.src[1], pa.dst[1], pa.ws[1].XR, t, sx, sz);
+}
+
 // blockIdx.y selects the system: K0 for the first, K1 for the second
 template <int K0, int K1, bool TAB>
 __global__ void __launch_bounds__(256)
@@ -717,20 +891,46 @@ __global__ void __launch_bounds__(256)
     col_ix_iz(D, col, ix, iz);
     g = penta_group(D, ix, iz);
   }
-  if (sys == 0) penta_line<K0, TAB>(D, col, ix, iz, g, lam, der, pa.src[0], pa.dst[0], pa.ws[0], pa.tab[0], sx, sz);
-  else penta_line<K1, TAB>(D, col, ix, iz, g, lam, der, pa.src[1], pa.dst[1], pa.ws[1], pa.tab[1], sx, sz);
+  if (sys == 0) penta_line<K0, TAB>(D, col, ix, iz, g, lam, der, pa.src[0], pa.dst[0], pa.ws[0], (const double4 *)pa.tab[0], sx, sz);
+  else penta_line<K1, TAB>(D, col, ix, iz, g, lam, der, pa.src[1], pa.dst[1], pa.ws[1], (const double4 *)pa.tab[1], sx, sz);
 }
+
+// Grids that take the whole factorisation.  It costs 72 B a row and group beside
+// the 64 B a row and column of the sweeps, and saves the pivots' chains: below
+// some 24,000 columns (375 wavefronts a system) those chains bound the solve,
+// above it the bytes.  k_penta with checkpoints -> k_penta_full, us: 32 x 65 x 32
+// 55 -> 22, 63 x 128 x 63 125 -> 52, 64 x 257 x 64 268 -> 110, 95 x 64 x 95 (18,336
+// columns) 69 -> 50, 128 x 257 x 128 (33,153) 361 -> 402.  The fused shift and
+// solve, whose chain is the longer: 32 x 65 x 32 86 -> 43, 64 x 128 x 64 209 -> 111,
+// 127 x 257 x 127 (32,640 columns) 575 -> 397, 160 x 200 x 160 (51,681) 519 -> 557.
+bool penta_full_tables(const Dims &D) { return D.ncol <= (D.exact ? 33000 : 24000); }
 
 size_t penta_table_bytes(const Dims &D) {
-  return (size_t)2 * ((D.ny - 2 + PC - 1) / PC) * (D.nx + 1) * (D.nz + 1) * sizeof(double4);
+  const size_t ng = (size_t)(D.nx + 1) * (D.nz + 1);
+  if (penta_full_tables(D)) return penta_full_bytes(D.ny - 2, ng);
+  return (size_t)2 * ((D.ny - 2 + PC - 1) / PC) * ng * sizeof(double4);
 }
 
-int launch_penta_factor(const Dims &D, int kind, double lambda, const double *der, void *tab, hipStream_t s) {
+int launch_penta_factor(const Dims &D, int nlam, const double *lambda, void *const *tabs, const double *der,
+                        hipStream_t s) {
+  if (nlam < 1 || nlam > 3) return hipErrorInvalidValue;
+  FactorArgs a;
+  for (int k = 0; k < nlam; k++) {
+    a.lam[k] = lambda[k];
+    a.tab[2 * k] = tabs[2 * k];
+    a.tab[2 * k + 1] = tabs[2 * k + 1];
+  }
   const int ng = (D.nx + 1) * (D.nz + 1);
-  dim3 grid((ng + 255) / 256);
-  if (kind == KD2V) hipLaunchKernelGGL(k_penta_factor<KD2V>, grid, dim3(256), 0, s, D, lambda, der, (double4 *)tab);
-  else if (kind == KETA) hipLaunchKernelGGL(k_penta_factor<KETA>, grid, dim3(256), 0, s, D, lambda, der, (double4 *)tab);
-  else return hipErrorInvalidValue;
+  dim3 grid((ng + 63) / 64, 2 * nlam);
+  const size_t lds = (size_t)D.ny * 20 * sizeof(double);
+  const bool cl = lds <= 65536;
+#define L(F, CLX) hipLaunchKernelGGL((k_penta_factor<F, CLX>), grid, dim3(64), CLX ? lds : 0, s, D, a, der)
+  if (penta_full_tables(D)) {
+    if (cl) L(true, 1); else L(true, 0);
+  } else {
+    if (cl) L(false, 1); else L(false, 0);
+  }
+#undef L
   return hipGetLastError();
 }
 
@@ -743,8 +943,13 @@ int launch_penta(const Dims &D, int nsys, const int *kinds, double lambda, const
     pa.src[k] = src[k];
     pa.dst[k] = dst[k];
     pa.ws[k] = ws[k];
-    pa.tab[k] = tabs ? (const double4 *)tabs[k] : nullptr;
+    pa.tab[k] = tabs ? tabs[k] : nullptr;
     if (!pa.tab[k]) tab = false;
+  }
+  if (tab && penta_full_tables(D)) {
+    if (nsys != 2 || kinds[0] != KD2V || kinds[1] != KETA) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_penta_full, dim3(pair_lanes(D) / 64, 2), dim3(64), 0, s, D, pa, lambda, der, sx, sz);
+    return hipGetLastError();
   }
   dim3 grid(((tab ? pair_lanes(D) : D.ncol) + 255) / 256, nsys);
 #define L(A, B, T) hipLaunchKernelGGL((k_penta<A, B, T>), grid, dim3(256), 0, s, D, pa, lambda, der, sx, sz)
@@ -1669,25 +1874,24 @@ int launch_shift_window(const Dims &D, int nq, void *const *q, const int *f32, d
 // elimination takes them.  Rows 0, 1 of x come from the reversed border
 // system, rows ny-2, ny-1 first from the record (for the ghost rows below row
 // 0), then from the back substitution.
-// Loads two rows ahead in each sweep, the phase factors of the second sweep
+// Loads two rows ahead in each sweep (four from the whole factorisation, whose
+// grids have registers to spare), the phase factors of the second sweep
 // with them (multiplied only where used: 5 % faster than carrying their
 // product, which made each prefetch wait for its loads).  Three wavefronts
 // per SIMD (168 VGPRs).  Deeper prefetch ran slower.
 // One system alone (half the launch) takes 0.48 of the time of both: the
 // kernel is bound by HBM bandwidth, not by the second, partly filled round.
-constexpr int SP_WAVES = 3, SP_PF = 2;
-#ifndef SP_LDS
-#define SP_LDS 1
-#endif
-template <int K>
+constexpr int SP_WAVES = 3, SP_PF = 2, SP_PFF = 4;
+template <int K, bool FULL>
 __device__ __forceinline__ void shift_penta_line(const Dims &D, int col, int ix, int iz, int g,
                                                  const D0Const &fcr,
                                                  const double *__restrict__ f0, const double *__restrict__ der,
                                                  const double2 *__restrict__ q, double2 *__restrict__ XRs,
                                                  const double2 *__restrict__ PX, const double2 *__restrict__ PZ,
                                                  double sx0s, double sz0s, double sx1s, double sz1s, double lam,
-                                                 double2 *__restrict__ XRp, const double4 *__restrict__ tab,
+                                                 double2 *__restrict__ XRp, const void *__restrict__ tab,
                                                  double2 *__restrict__ dst) {
+  constexpr int PF = FULL ? SP_PFF : SP_PF;
   const size_t nc = D.ncol, ws = D.ncs;  // field rows, workspace rows
   const int m = D.ny, mi = m - 2;
   if (ix == 0 && iz == 0 && K == KD2V) {  // the (0,0) D2V line is zero (src/hst_linsolve.f90:199,221-224)
@@ -1696,7 +1900,7 @@ __device__ __forceinline__ void shift_penta_line(const Dims &D, int col, int ix,
   }
   // 1. the reversed D0 elimination: reversed row k is row m-1-k
   C x1{0, 0}, x2{0, 0}, sx0{0, 0}, sx1{0, 0};
-  rows_ascending<SP_PF, C>(
+  rows_ascending<PF, C, FULL>(
       mi, [&](int k) { return ld(q + (size_t)(m - 1 - k + 2) * nc + col); },
       [&](int k, const C &v) {
         C bx = v;
@@ -1730,6 +1934,8 @@ __device__ __forceinline__ void shift_penta_line(const Dims &D, int col, int ix,
   const double al = D.alfa0 * ix, be = D.beta0 * iz;
   const double kk = al * al + be * be, ni = D.ni;
   PentaFactor f;
+  const size_t ng = (size_t)(D.nx + 1) * (D.nz + 1);
+  const PentaFull ft = penta_full_view((void *)tab, mi, ng);
   C px1{0, 0}, px2{0, 0}, psx0{0, 0}, psx1{0, 0}, r25p{0, 0}, r27p{0, 0};
   // row i (< mi) of the elimination
   auto feed = [&](int i, const C &bin) {
@@ -1763,33 +1969,55 @@ __device__ __forceinline__ void shift_penta_line(const Dims &D, int col, int ix,
   // waited for one row after another
   struct Row {
     C xr, px, pz;
+    double4 f;  // FULL: the factors of the row of the line solve that this one completes
+    double v;
   };
   C xk1 = b1, xk2 = b2;
-  rows_descending<SP_PF, Row>(
+  rows_descending<PF, Row, FULL>(
       mi,
       [&](int k) {
         const int i = m - 1 - k;
-        return Row{ld(XRs + (size_t)k * ws + col), ld(PX + (size_t)i * D.NXm + ix),
-                   ld(PZ + (size_t)i * D.NZm + az + D.nz)};
+        Row r{ld(XRs + (size_t)k * ws + col), ld(PX + (size_t)i * D.NXm + ix),
+              ld(PZ + (size_t)i * D.NZm + az + D.nz), make_double4(0, 0, 0, 0), 0.0};
+        if constexpr (FULL) {
+          r.f = ft.f[ng * (i - 2) + g];
+          r.v = ft.v[ng * (i - 2) + g];
+        }
+        return r;
       },
       [&](int k, const Row &r) {
         const C xk = r.xr - F0(k, 5) * yb1 - F0(k, 6) * yb2 - F0(k, 3) * xk1 - F0(k, 4) * xk2;
         xk2 = xk1;
         xk1 = xk;
         const int i = m - 1 - k - 2;  // x'(m-1-k) completes row m-3-k < mi
-        feed(i, reweight(i, xk * (r.px * (iz < 0 ? conj(r.pz) : r.pz))));
+        const C bin = reweight(i, xk * (r.px * (iz < 0 ? conj(r.pz) : r.pz)));
+        if constexpr (FULL) {
+          const C bx = (bin - r.f.x * px2 - r.f.y * px1) * r.f.z;
+          st(XRp + (size_t)i * ws + col, bx);
+          psx0 = psx0 + r.f.w * bx;
+          psx1 = psx1 + r.v * bx;
+          px2 = px1;
+          px1 = bx;
+        } else {
+          feed(i, bin);
+        }
       });
   // the border rows' right-hand sides (the loop above covers the rows < mi,
   // so that its body has no branch on the row)
   r25p = reweight(m - 2, xp0 * ph1);  // x'(m) = x'(0) ph1
   r27p = reweight(m - 1, xp1 * ph1);  // x'(m+1) = x'(1) ph1
   // 3. the line solve's border system and back substitution (as penta_line)
-  double rq[25];
+  double rq[25], u21;
+  if constexpr (FULL) {
+    u21 = penta_record(ft, ng, g, rq);
+  } else {
   rq[3] = f.sp0; rq[4] = f.sq0; rq[5] = f.w2 * f.u22 + f.w1 * f.u11; rq[6] = f.w1 * f.u12;
   rq[9] = f.sp1; rq[10] = f.sq1; rq[11] = f.v2 * f.u22 + f.v1 * f.u11; rq[12] = f.v1 * f.u12;
   rq[15] = f.p2 - f.u21 * f.p1; rq[16] = f.q2 - f.u21 * f.q1; rq[17] = f.u22 - f.u21 * f.u11; rq[18] = -f.u21 * f.u12;
   rq[21] = f.p1; rq[22] = f.q1; rq[23] = f.u11; rq[24] = f.u12;
-  const C xm2 = px2 - f.u21 * px1, xm1 = px1;
+  u21 = f.u21;
+  }
+  const C xm2 = px2 - u21 * px1, xm1 = px1;
   const int ga = m - 2;
   C c1, c2;
   border_solve(rq, coefk<K>(lam, ni, kk, der, ga, -2), coefk<K>(lam, ni, kk, der, ga, -1),
@@ -1802,37 +2030,30 @@ __device__ __forceinline__ void shift_penta_line(const Dims &D, int col, int ix,
   st(dst + (size_t)(m - 1 + 2) * nc + col, c2);
   const C cph1 = conj(ph1);
   const C zb1 = cph1 * c1, zb2 = cph1 * c2;
+  if constexpr (FULL) {
+    penta_full_back(D, col, g, ft, zb1, zb2, c1, c2, XRp, ws, dst);
+    return;
+  }
   penta_back<K>(
-      D, g, lam, kk, der, tab, zb1, zb2, c1, c2, [&](int i) { return ld(XRp + (size_t)i * ws + col); },
+      D, g, lam, kk, der, (const double4 *)tab, zb1, zb2, c1, c2, [&](int i) { return ld(XRp + (size_t)i * ws + col); },
       [&](int i, const C &x) { st(dst + (size_t)(i + 2) * nc + col, x); });
 }
 
 struct ShiftPentaArgs {
   const double2 *q[2];
   double2 *xrs[2], *xrp[2], *dst[2];
-  const double4 *tab[2];
+  const void *tab[2];
 };
 
 // blockIdx.y: system 0 (D2V on rhs2) or 1 (ETA on rhs1)
 // CL: the reversed D0 factor rows read from a copy in LDS (9 doubles a row)
-template <int CL>
-__global__ void __launch_bounds__(256, SP_WAVES)
+template <int CL, bool FULL, int NT>
+__global__ void __launch_bounds__(NT, FULL ? 1 : SP_WAVES)
     k_shift_penta(Dims D, ShiftPentaArgs a, D0Const fcr, const double *__restrict__ f0g,
                   const double *__restrict__ der, const double2 *__restrict__ PX, const double2 *__restrict__ PZ,
                   double sx0s, double sz0s, double sx1s, double sz1s, double lam) {
   extern __shared__ double f0s[];
-  if constexpr (CL) {
-    const int n = (D.ny - 2) * 9;
-    for (int b0 = 0; b0 < n; b0 += 16 * 256) {
-      double v[16];
-#pragma unroll
-      for (int u = 0; u < 16; u++) v[u] = f0g[min(b0 + u * 256 + (int)threadIdx.x, n - 1)];
-#pragma unroll
-      for (int u = 0; u < 16; u++)
-        if (b0 + u * 256 + (int)threadIdx.x < n) f0s[b0 + u * 256 + threadIdx.x] = v[u];
-    }
-    __syncthreads();
-  }
+  if constexpr (CL) rows_to_lds<NT>(f0s, f0g, (D.ny - 2) * 9);
   const double *const f0r = CL ? f0s : f0g;
   // one column per lane in column order: a wavefront's row is one run of 64
   // columns (the +iz, -iz pairs of pair_lane share the table rows but read two
@@ -1845,10 +2066,10 @@ __global__ void __launch_bounds__(256, SP_WAVES)
   col_ix_iz(D, col, ix, iz);
   const int g = penta_group(D, ix, iz);
   if (sys == 0)
-    shift_penta_line<KD2V>(D, col, ix, iz, g, fcr, f0r, der, a.q[0], a.xrs[0], PX, PZ, sx0s, sz0s, sx1s, sz1s, lam, a.xrp[0],
+    shift_penta_line<KD2V, FULL>(D, col, ix, iz, g, fcr, f0r, der, a.q[0], a.xrs[0], PX, PZ, sx0s, sz0s, sx1s, sz1s, lam, a.xrp[0],
                            a.tab[0], a.dst[0]);
   else
-    shift_penta_line<KETA>(D, col, ix, iz, g, fcr, f0r, der, a.q[1], a.xrs[1], PX, PZ, sx0s, sz0s, sx1s, sz1s, lam, a.xrp[1],
+    shift_penta_line<KETA, FULL>(D, col, ix, iz, g, fcr, f0r, der, a.q[1], a.xrs[1], PX, PZ, sx0s, sz0s, sx1s, sz1s, lam, a.xrp[1],
                            a.tab[1], a.dst[1]);
 }
 
@@ -1863,16 +2084,18 @@ int launch_shift_penta(const Dims &D, const double2 *q2, const double2 *q1, doub
   for (int k = 0; k < 2; k++) {
     a.xrs[k] = xrs[k];
     a.xrp[k] = xrp[k];
-    a.tab[k] = (const double4 *)tabs[k];
+    a.tab[k] = tabs[k];
   }
-  dim3 grid((D.ncol + 255) / 256, 2);
   const size_t lds = (size_t)(D.ny - 2) * 9 * sizeof(double);
-  if (SP_LDS && lds <= 49152)
-    hipLaunchKernelGGL(k_shift_penta<1>, grid, dim3(256), lds, s, D, a, fcr, f0r, der, PX, PZ, sx0, sz0, sx1, sz1,
-                       lambda);
-  else
-    hipLaunchKernelGGL(k_shift_penta<0>, grid, dim3(256), 0, s, D, a, fcr, f0r, der, PX, PZ, sx0, sz0, sx1, sz1,
-                       lambda);
+#define L(CLX, F, NT)                                                                                             \
+  hipLaunchKernelGGL((k_shift_penta<CLX, F, NT>), dim3((D.ncol + NT - 1) / NT, 2), dim3(NT), CLX ? lds : 0, s, D, a, \
+                     fcr, f0r, der, PX, PZ, sx0, sz0, sx1, sz1, lambda)
+  if (penta_full_tables(D)) {
+    if (lds <= 49152) L(1, true, 64); else L(0, true, 64);
+  } else {
+    if (lds <= 49152) L(1, false, 256); else L(0, false, 256);
+  }
+#undef L
   return hipGetLastError();
 }
 
