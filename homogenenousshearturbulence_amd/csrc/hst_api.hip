@@ -674,13 +674,15 @@ static int recover(bool compact, double sx, double sz) {
       });
     else
       rc = run("dvdy", 4.0 * bytes_field(), [&] {
-        return launch_d0solve(S.D, 1, 0, S.F[HST_V2], S.F[HST_V3], nullptr, S.XR[0], S.d_f0, S.fc, S.d_der,
-                              S.d_dyl, sx, sz, nullptr, nullptr, S.stream);
+        const double2 *v[1] = {S.F[HST_V2]};
+        return launch_d0solve(S.D, 1, 0, 1, v, &S.F[HST_V3], nullptr, S.XR, S.d_f0, S.fc, S.d_der, S.d_dyl, sx, sz,
+                              nullptr, nullptr, S.stream);
       });
   } else {
     rc = run("dy_recover", 6.0 * bytes_field(), [&] {
-      return launch_d0solve(S.D, 1, 1, S.F[HST_V2], S.F[HST_V1], S.F[HST_V3], S.XR[0], S.d_f0, S.fc, S.d_der,
-                            S.d_dyl, sx, sz, nullptr, nullptr, S.stream);
+      const double2 *v[1] = {S.F[HST_V2]};
+      return launch_d0solve(S.D, 1, 1, 1, v, &S.F[HST_V1], S.F[HST_V3], S.XR, S.d_f0, S.fc, S.d_der, S.d_dyl, sx, sz,
+                            nullptr, nullptr, S.stream);
     });
   }
   if (rc) return rc;
@@ -956,11 +958,12 @@ int hst_gpu_init(const hst_deck *deck, int precision) {
     if (dy_window_setup(sig)) {
       HIPCHK(hipMalloc(&S.d_sig, sig.size() * sizeof(double)));
       HIPCHK(hipMemcpy(S.d_sig, sig.data(), sig.size() * sizeof(double), hipMemcpyHostToDevice));
-      S.dyw = !off("HST_NO_DYWIN");
+      S.dyw = !off("HST_NO_DYWIN") && dy_one_sweep(D);
       S.shw = !off("HST_NO_SHWIN");
     }
   }
-  S.part_cap = std::max<size_t>((size_t)D.NYg * D.nzd, (size_t)((D.ncol + 255) / 256) * NSTAT + 64);
+  // the CFL maxima of the x pass's blocks, or the statistics' sums per block
+  S.part_cap = std::max<size_t>((size_t)D.NYg * D.nzd, (size_t)((D.ncol + 63) / 64) * (NSTAT + 9) + 64);
   HIPCHK(hipMalloc(&S.d_part, S.part_cap * sizeof(double)));
   HIPCHK(hipHostMalloc((void **)&S.h_part, S.part_cap * sizeof(double), hipHostMallocDefault));
   if (make_fft_tables(D, S.mixed, &S.tables)) return fail("twiddle tables");
@@ -1226,8 +1229,9 @@ int hst_gpu_line_solve(int kind, double lambda, int src, int dst, double shift_x
   if (src == dst) return fail("line_solve: src and dst must be different fields");
   if (kind == HST_KIND_D0 || kind == HST_KIND_DY) {
     return run(kind == HST_KIND_D0 ? "d0_solve" : "dy_solve", 4.0 * bytes_field(), [&] {
-      return launch_d0solve(S.D, kind == HST_KIND_DY ? 1 : 0, 0, S.F[src], S.F[dst], nullptr, S.XR[0], S.d_f0, S.fc,
-                            S.d_der, S.d_dyl, shift_x, shift_z, nullptr, nullptr, S.stream);
+      const double2 *f[1] = {S.F[src]};
+      return launch_d0solve(S.D, kind == HST_KIND_DY ? 1 : 0, 0, 1, f, &S.F[dst], nullptr, S.XR, S.d_f0, S.fc, S.d_der,
+                            S.d_dyl, shift_x, shift_z, nullptr, nullptr, S.stream);
     });
   }
   if (kind < 1 || kind > 3) return fail("unknown system kind");
@@ -1354,32 +1358,32 @@ int hst_gpu_outstats(double time, double out[10]) {
     a.inlayer = S.d_inlayer;
     a.inc00 = 0;  // the (0,0) column is the imposed layer: mean flow
   }
-  int nb = 0;
+  // the sums of the fields and of their y derivatives: two launches, one copy
+  int nb = 0, np = 0;
   int rc = run("stats", 3.0 * bytes_field(), [&] {
     return launch_stats(S.D, a, S.F[1], S.F[2], S.F[3], S.d_dyl, S.d_part, &nb, S.exz_acc, S.stream);
   });
   if (rc) return rc;
-  std::vector<double> h((size_t)nb * NSTAT);
-  HIPCHK(hipMemcpyAsync(h.data(), S.d_part, h.size() * sizeof(double), hipMemcpyDeviceToHost, S.stream));
+  double sx, sz;
+  shear_shifts(time, sx, sz);
+  double *dpart = S.d_part + (size_t)nb * NSTAT;
+  rc = run("dy_stats", 3.0 * 3.0 * bytes_field(), [&] {
+    const double2 *v[3] = {S.F[1], S.F[2], S.F[3]};
+    return launch_d0solve(S.D, 1, 2, 3, v, nullptr, nullptr, S.XR, S.d_f0, S.fc, S.d_der, S.d_dyl, sx, sz, dpart, &np,
+                          S.stream, a.inlayer, a.inc00 ? 0 : 1);
+  });
+  if (rc) return rc;
+  const size_t n = (size_t)nb * NSTAT + (size_t)np * 3;
+  HIPCHK(hipMemcpyAsync(S.h_part, S.d_part, n * sizeof(double), hipMemcpyDeviceToHost, S.stream));
   HIPCHK(hipStreamSynchronize(S.stream));
   double s[NSTAT] = {0};
   for (int b = 0; b < nb; b++)
-    for (int k = 0; k < NSTAT; k++) s[k] += h[(size_t)b * NSTAT + k];
-  double sx, sz;
-  shear_shifts(time, sx, sz);
+    for (int k = 0; k < NSTAT; k++) s[k] += S.h_part[(size_t)b * NSTAT + k];
   double eps = s[6], e_in = s[11], e_out = s[12];
-  for (int c = 1; c <= 3; c++) {
-    int np = 0;
-    rc = run("dy_stats", 3.0 * bytes_field(), [&] {
-      return launch_d0solve(S.D, 1, 2, S.F[c], nullptr, nullptr, S.XR[0], S.d_f0, S.fc, S.d_der, S.d_dyl, sx, sz,
-                            S.d_part, &np, S.stream, a.inlayer, a.inc00 ? 0 : 1);
-    });
-    if (rc) return rc;
-    std::vector<double> g((size_t)np * 3);
-    HIPCHK(hipMemcpyAsync(g.data(), S.d_part, g.size() * sizeof(double), hipMemcpyDeviceToHost, S.stream));
-    HIPCHK(hipStreamSynchronize(S.stream));
+  const double *g = S.h_part + (size_t)nb * NSTAT;
+  for (int c = 0; c < 3; c++) {
     double grad = 0.0, g_in = 0.0, g_out = 0.0;
-    for (int b = 0; b < np; b++) {
+    for (int b = c * (np / 3); b < (c + 1) * (np / 3); b++) {
       grad += g[(size_t)b * 3];
       g_in += g[(size_t)b * 3 + 1];
       g_out += g[(size_t)b * 3 + 2];

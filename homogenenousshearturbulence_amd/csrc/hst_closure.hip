@@ -767,7 +767,7 @@ struct hst_closure {
   void *tables = nullptr;  // FP64 tables of the solver's z forward transform
   double2 *fields = nullptr;  // 15 coarse fields: U[3], Pbar[6], Tau[6]
   double2 *Gy = nullptr;      // 3 y derivatives
-  double2 *XR = nullptr;      // D0 solve workspace
+  double2 *XR = nullptr;      // the workspaces of the three D0 solves
   Cx<double> *Hc = nullptr;   // z-inverse output, 18 fields
   double *phys = nullptr;     // 18 physical fields of the interior rows
   double2 *stage = nullptr;   // layout staging, one field
@@ -849,11 +849,14 @@ int filter_weights(int nyf, int nyc, std::vector<int> &j0, std::vector<double> &
 // fields to physical values: phys fields 0..8 (and 9..17)
 int to_physical(hst_closure *c, const double2 *const U[3], bool sample, double sx, double sz, hipStream_t st) {
   const Dims &D = c->D;
+  double2 *Gy[3], *XR[3];
   for (int i = 0; i < 3; i++) {
-    int rc = launch_d0solve(D, 1, 0, U[i], c->Gy + (size_t)i * c->nf(), nullptr, c->XR, c->d_f0, c->fc, c->d_der,
-                            c->d_dyl, sx, sz, nullptr, nullptr, st);
-    if (rc) return cfail("y derivative", rc);
+    Gy[i] = c->Gy + (size_t)i * c->nf();
+    XR[i] = c->XR + (size_t)i * (D.ny - 2) * D.ncol;
   }
+  if (int rc = launch_d0solve(D, 1, 0, 3, U, Gy, nullptr, XR, c->d_f0, c->fc, c->d_der, c->d_dyl, sx, sz, nullptr,
+                              nullptr, st))
+    return cfail("y derivatives", rc);
   ZSrc zs;
   int nf = 0;
   for (int i = 0; i < 3; i++) {
@@ -1024,7 +1027,7 @@ int hst_closure_create(const hst_deck *coarse, int64_t capacity, hst_closure **o
   MAL(c->fields, 15 * c->nf() * sizeof(double2));
   MAL(c->Gy, 3 * c->nf() * sizeof(double2));
   MAL(c->stage, c->nf() * sizeof(double2));
-  MAL(c->XR, (size_t)(D.ny - 2) * D.ncol * sizeof(double2));
+  MAL(c->XR, 3 * (size_t)(D.ny - 2) * D.ncol * sizeof(double2));
   MAL(c->Hc, 18 * (size_t)D.ny * D.nzd * D.NXp * sizeof(Cx<double>));
   MAL(c->phys, 18 * c->fs() * sizeof(double));
   (void)hipMemset(c->fields, 0, 15 * c->nf() * sizeof(double2));

@@ -117,16 +117,18 @@ size_t penta_table_bytes(const Dims &D);
 int launch_penta_factor(const Dims &D, int nlam, const double *lambda, void *const *tabs, const double *der,
                         hipStream_t s);
 
-// D0-type solves with the shared factorisation.  rhs_mode 0: D0 x = src;
-// 1: D0 x = D1 src (src ghost rows filled).  out_mode 0: x into dst;
-// 1: u, w recovered from x = dv/dy and eta (dst = V1 holding eta, dst3 = V3);
-// 2: sums of w |x|^2 into part, three doubles per block: all rows, the rows
+// D0-type solves with the shared factorisation of nf (1..3) fields in one
+// launch.  rhs_mode 0: D0 x = src; 1: D0 x = D1 src (src ghost rows filled).
+// out_mode 0: x into dst; 1 (rhs_mode 1, one field): u, w recovered from
+// x = dv/dy and eta (dst = V1 holding eta, dst3 = V3); 2 (rhs_mode 1): sums of
+// w |x|^2 into part, three doubles per block, field by field: all rows, the rows
 // with inlayer set, the others (inlayer may be null: every row outside); the
-// (0,0) column is left out when skip00 is set.
-int launch_d0solve(const Dims &D, int rhs_mode, int out_mode, const double2 *src, double2 *dst, double2 *dst3,
-                   double2 *XR, const double *f0rows, const D0Const &fc, const double *der, const double *dyl,
-                   double sx, double sz, double *part, int *n_part, hipStream_t s, const int *inlayer = nullptr,
-                   int skip00 = 0);
+// (0,0) column is left out when skip00 is set.  XR: a workspace of ny - 2 rows
+// per field.
+int launch_d0solve(const Dims &D, int rhs_mode, int out_mode, int nf, const double2 *const *src, double2 *const *dst,
+                   double2 *dst3, double2 *const *XR, const double *f0rows, const D0Const &fc, const double *der,
+                   const double *dyl, double sx, double sz, double *part, int *n_part, hipStream_t s,
+                   const int *inlayer = nullptr, int skip00 = 0);
 // D0 x = D1 src in one sweep (OUT 0 of launch_d0solve, the time step's dv/dy)
 // with the back substitution windowed over dy_window_rows() rows; sig holds
 // the back substitution of -B1, -B2 over the first dy_window_rows() rows
@@ -134,6 +136,7 @@ int launch_d0solve(const Dims &D, int rhs_mode, int out_mode, const double2 *src
 int launch_dy_window(const Dims &D, const double2 *src, double2 *dst, const double *f0rows, const D0Const &fc,
                      const double *der, const double *sig, double sx, double sz, hipStream_t s);
 int dy_window_rows();
+bool dy_one_sweep(const Dims &D);  // whether that is the faster on this grid
 // batched FP64 line transforms of the per-field entry points (hst_lines.hip)
 int launch_cfft_lines(int n, int sign, double2 *data, int64_t nlines, const void *tw, hipStream_t s);
 int launch_rfft_lines(int m, int dir, double2 *data, int64_t nlines, const void *tw, const void *twh,

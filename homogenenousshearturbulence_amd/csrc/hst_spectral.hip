@@ -734,7 +734,7 @@ __device__ __forceinline__ void penta_full_back(const Dims &D, int col, int g, c
 // one slab): forward elimination of rows 0..ny-3 with the rows generated from
 // der, record in registers, 2x2 border system, back substitution.  With a
 // factor table the workspace holds only the eliminated right-hand side.
-template <int K, bool TAB>
+template <int K, bool TAB, int PFW = PF_PENTA, int PFV = PF_BWD>
 __device__ __forceinline__ void penta_line(const Dims &D, int col, int ix, int iz, int g, double lam,
                                            const double *__restrict__ der, const double2 *__restrict__ src,
                                            double2 *__restrict__ dst, const PentaWS &ws,
@@ -750,7 +750,7 @@ __device__ __forceinline__ void penta_line(const Dims &D, int col, int ix, int i
   const double kk = al * al + be * be, ni = D.ni;
   PentaFactor f;
   C x1{0, 0}, x2{0, 0}, sx0{0, 0}, sx1{0, 0};
-  rows_ascending<PF_PENTA, C>(
+  rows_ascending<PFW, C>(
       mi, [&](int i) { return ld(src + (size_t)(i + 2) * nc + col); },
       [&](int i, const C &bin) {
         double l2, l1, rp, t1, t2, p, q;
@@ -793,7 +793,7 @@ __device__ __forceinline__ void penta_line(const Dims &D, int col, int ix, int i
         [&](int i, const C &x) { st(dst + (size_t)(i + 2) * nc + col, x); });
   } else {
     C xk1 = b1, xk2 = b2;
-    rows_descending<PF_BWD, WSRow>(
+    rows_descending<PFV, WSRow>(
         mi,
         [&](int i) {
           const size_t o = (size_t)i * nc + col;
@@ -968,13 +968,43 @@ int launch_penta(const Dims &D, int nsys, const int *kinds, double lambda, const
 // rows table: [i][L2 L1 RP U1 U2 B1 B2 W V]
 #define F0(i, k) f0[(i) * 9 + (k)]
 
-// Forward sweep of D0 x = r for one lane, XR stored; r = src (RHS 0) or the
+// The coefficients of a row of the D0 solves: the D1 taps (row i < ny) and the
+// columns of the factorisation (i < ny - 2), from a copy in LDS (CL, by
+// d0_rows_to_lds) or from global memory.
+constexpr int D0C = 14;
+template <int CL>
+struct D0Rows {
+  const double *lds, *f0, *der;
+  __device__ __forceinline__ double tap(int i, int t) const {
+    return CL ? lds[i * D0C + t + 2] : DER(der, i, 1, t);
+  }
+  __device__ __forceinline__ double f(int i, int k) const { return CL ? lds[i * D0C + 5 + k] : F0(i, k); }
+};
+template <int NT>
+__device__ __forceinline__ void d0_rows_to_lds(double *lds, const double *__restrict__ f0,
+                                               const double *__restrict__ der, int ny) {
+  const int n = ny * D0C, nf = (ny - 2) * 9;
+  for (int b0 = 0; b0 < n; b0 += 16 * NT) {
+    double v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      const int k = min(b0 + u * NT + (int)threadIdx.x, n - 1), i = k / D0C, j = k - i * D0C;
+      v[u] = j < 5 ? DER(der, i, 1, j - 2) : f0[min(i * 9 + j - 5, nf - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; u++)
+      if (b0 + u * NT + (int)threadIdx.x < n) lds[b0 + u * NT + threadIdx.x] = v[u];
+  }
+  __syncthreads();
+}
+static size_t d0_lds_bytes(int ny) { return (size_t)ny * D0C * sizeof(double); }
+
+// Forward sweep of D0 x = r for one lane, the eliminated rows to xr, xs apart; r = src (RHS 0) or the
 // D1 stencil of src (RHS 1, ghost rows filled).  Also returns the border
 // rows' right-hand sides r(ny-2), r(ny-1).
-template <int RHS, typename ST = double2, typename XT = double2>
-__device__ __forceinline__ void d0_forward(const Dims &D, const double *__restrict__ f0,
-                                           const double *__restrict__ der, const ST *__restrict__ src,
-                                           XT *__restrict__ XR, int col, C &x1, C &x2, C &sx0, C &sx1, C &r25,
+template <int RHS, int CL>
+__device__ __forceinline__ void d0_forward(const Dims &D, const D0Rows<CL> &co, const double2 *__restrict__ src,
+                                           double2 *xr, size_t xs, int col, C &x1, C &x2, C &sx0, C &sx1, C &r25,
                                            C &r27) {
   const size_t nc = D.ncol;
   const int m = D.ny, mi = m - 2;
@@ -987,7 +1017,7 @@ __device__ __forceinline__ void d0_forward(const Dims &D, const double *__restri
   auto stencil = [&](int i) {
     C r{0, 0};
 #pragma unroll
-    for (int j = -2; j <= 2; j++) r = r + DER(der, i, 1, j) * w[j + 2];
+    for (int j = -2; j <= 2; j++) r = r + co.tap(i, j) * w[j + 2];
     return r;
   };
   auto push = [&](const C &v) {
@@ -1003,12 +1033,13 @@ __device__ __forceinline__ void d0_forward(const Dims &D, const double *__restri
           push(v);
           bx = stencil(i);
         }
-        if (i >= 2) bx = bx - F0(i, 0) * x2;
-        if (i >= 1) bx = bx - F0(i, 1) * x1;
-        bx = bx * F0(i, 2);
-        st(XR + (size_t)i * nc + col, bx);
-        sx0 = sx0 + F0(i, 7) * bx;
-        sx1 = sx1 + F0(i, 8) * bx;
+        // (the multipliers of rows that are not there are zero)
+        bx = bx - co.f(i, 0) * x2;
+        bx = bx - co.f(i, 1) * x1;
+        bx = bx * co.f(i, 2);
+        st(xr + i * xs, bx);
+        sx0 = sx0 + co.f(i, 7) * bx;
+        sx1 = sx1 + co.f(i, 8) * bx;
         x2 = x1;
         x1 = bx;
       });
@@ -1033,13 +1064,28 @@ __device__ __forceinline__ void d0_border(const D0Const &fc, C ph, C x1, C x2, C
 // D0 x = src (RHS 0) or D0 x = D1 src (RHS 1); OUT 0: x to dst; 1: recover
 // u, w from x = dv/dy and eta = dst (src/hst_equations.f90:303-324); 2: block
 // sums of w |x|^2 (the dissipation's y derivatives, src/hst_stats.f90:200-223).
-template <int RHS, int OUT>
-__global__ void __launch_bounds__(256)
+// blockIdx.y: the field of the list.  NT = 64 on grids whose wavefronts do not
+// fill the chip, the back substitution eight rows ahead there.  Read as scalar
+// loads, the coefficients were waited for row by row: 32 x 65 x 32 46 -> 23 us,
+// 95 x 64 x 95 60 -> 29 us; the three fields of the statistics in one launch
+// 96 x 193 x 96 3 x 199 -> 170 us.
+struct D0List {
+  const double2 *src[3];
+  double2 *dst[3], *XR[3];
+};
+template <int RHS, int OUT, int CL, int NT>
+__global__ void __launch_bounds__(NT)
     k_d0solve(Dims D, D0Const fc, const double *__restrict__ f0, const double *__restrict__ der,
-              const double *__restrict__ dyl, const double2 *__restrict__ src, double2 *__restrict__ dst,
-              double2 *__restrict__ dst3, double2 *__restrict__ XR, double sx, double sz, double *__restrict__ part,
-              const int *__restrict__ inlayer, int skip00) {
-  const int col = blockIdx.x * blockDim.x + threadIdx.x;
+              const double *__restrict__ dyl, D0List fl, double2 *__restrict__ dst3, double sx, double sz,
+              double *__restrict__ part, const int *__restrict__ inlayer, int skip00) {
+  extern __shared__ double cfs[];
+  if constexpr (CL) d0_rows_to_lds<NT>(cfs, f0, der, D.ny);
+  const D0Rows<CL> co{cfs, f0, der};
+  constexpr int PFB = NT == 64 ? 8 : PF_BWD;
+  const double2 *__restrict__ src = fl.src[blockIdx.y];
+  double2 *__restrict__ dst = fl.dst[blockIdx.y];
+  double2 *__restrict__ XR = fl.XR[blockIdx.y];
+  const int col = blockIdx.x * NT + threadIdx.x;
   const bool act = col < D.ncol;
   const int cl = act ? col : 0;
   int ix, iz;
@@ -1050,7 +1096,7 @@ __global__ void __launch_bounds__(256)
   const bool skip = skip00 && ix == 0 && iz == 0;
   if (act) {
     C x1, x2, sx0, sx1, r25, r27;
-    d0_forward<RHS>(D, f0, der, src, XR, col, x1, x2, sx0, sx1, r25, r27);
+    d0_forward<RHS, CL>(D, co, src, XR + col, nc, col, x1, x2, sx0, sx1, r25, r27);
     const C ph = cexpi(-(D.alfa0 * ix * sx + D.beta0 * iz * sz));
     C b1, b2;
     d0_border(fc, ph, x1, x2, sx0, sx1, r25, r27, b1, b2);
@@ -1085,17 +1131,17 @@ __global__ void __launch_bounds__(256)
     struct Row {
       C xr, eta;
     };
-    rows_descending<PF_BWD, Row>(
+    rows_descending<PFB, Row>(
         m - 2, [&](int i) { return Row{ld(XR + (size_t)i * nc + col), eta_at(i)}; },
         [&](int i, const Row &r) {
-          const C xk = r.xr - F0(i, 5) * yb1 - F0(i, 6) * yb2 - F0(i, 3) * xk1 - F0(i, 4) * xk2;
+          const C xk = r.xr - co.f(i, 5) * yb1 - co.f(i, 6) * yb2 - co.f(i, 3) * xk1 - co.f(i, 4) * xk2;
           emit(i, xk, r.eta);
           xk2 = xk1;
           xk1 = xk;
         });
   }
   if constexpr (OUT == 2) {
-    __shared__ double red[3][4];
+    __shared__ double red[3][NT / 64];
     double v[3] = {acc, ain, aout};
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -1105,25 +1151,50 @@ __global__ void __launch_bounds__(256)
     __syncthreads();
     if (threadIdx.x < 3) {
       const int k = threadIdx.x;
-      part[(size_t)blockIdx.x * 3 + k] = red[k][0] + red[k][1] + red[k][2] + red[k][3];
+      double t = red[k][0];
+      for (int w = 1; w < NT / 64; w++) t += red[k][w];
+      part[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 3 + k] = t;
     }
   }
 }
 
-int launch_d0solve(const Dims &D, int rhs_mode, int out_mode, const double2 *src, double2 *dst, double2 *dst3,
-                   double2 *XR, const double *f0rows, const D0Const &fc, const double *der, const double *dyl,
-                   double sx, double sz, double *part, int *n_part, hipStream_t s, const int *inlayer, int skip00) {
-  dim3 grid((D.ncol + 255) / 256);
-  if (n_part) *n_part = grid.x;
-#define L(R, O)                                                                                                 \
-  hipLaunchKernelGGL((k_d0solve<R, O>), grid, dim3(256), 0, s, D, fc, f0rows, der, dyl, src, dst, dst3, XR, sx, sz, \
-                     part, inlayer, skip00)
-  if (rhs_mode == 0) {
-    if (out_mode == 0) L(0, 0); else if (out_mode == 1) L(0, 1); else L(0, 2);
-  } else {
-    if (out_mode == 0) L(1, 0); else if (out_mode == 1) L(1, 1); else L(1, 2);
+// A column kernel's block: one wavefront where nsys systems of the grid's columns
+// make fewer wavefronts than the chip has SIMDs (each then has a CU's caches, LDS
+// and memory path nearly to itself), four above.
+static bool small_columns(const Dims &D, int nsys) { return (long long)D.ncol * nsys <= 64 * 1024; }
+
+int launch_d0solve(const Dims &D, int rhs_mode, int out_mode, int nf, const double2 *const *src, double2 *const *dst,
+                   double2 *dst3, double2 *const *XR, const double *f0rows, const D0Const &fc, const double *der,
+                   const double *dyl, double sx, double sz, double *part, int *n_part, hipStream_t s,
+                   const int *inlayer, int skip00) {
+  if (nf < 1 || nf > 3) return hipErrorInvalidValue;
+  D0List fl;
+  for (int k = 0; k < nf; k++) {
+    fl.src[k] = src[k];
+    fl.dst[k] = dst ? dst[k] : nullptr;
+    fl.XR[k] = XR[k];
   }
+  const bool small = small_columns(D, nf);
+  const int nt = small ? 64 : 256;
+  const size_t lds = d0_lds_bytes(D.ny);
+  const bool cl = lds <= 65536;
+  dim3 grid((D.ncol + nt - 1) / nt, nf);
+  if (n_part) *n_part = grid.x * grid.y;
+#define L4(R, O, CLX, NT)                                                                                        \
+  hipLaunchKernelGGL((k_d0solve<R, O, CLX, NT>), grid, dim3(NT), CLX ? lds : 0, s, D, fc, f0rows, der, dyl, fl, dst3, \
+                     sx, sz, part, inlayer, skip00)
+#define L(R, O)                                                 \
+  do {                                                          \
+    if (small) { if (cl) L4(R, O, 1, 64); else L4(R, O, 0, 64); } \
+    else { if (cl) L4(R, O, 1, 256); else L4(R, O, 0, 256); }   \
+  } while (0)
+  if (rhs_mode == 0 && out_mode == 0) L(0, 0);
+  else if (rhs_mode == 1 && out_mode == 0) L(1, 0);
+  else if (rhs_mode == 1 && out_mode == 1 && nf == 1) L(1, 1);
+  else if (rhs_mode == 1 && out_mode == 2) L(1, 2);
+  else return hipErrorInvalidValue;
 #undef L
+#undef L4
   return hipGetLastError();
 }
 
@@ -1293,9 +1364,73 @@ __global__ void __launch_bounds__(256, 2)
     st(dst + (size_t)(i + 2) * nc + col, fx[i] + sig[2 * i] * yb1 + sig[2 * i + 1] * yb2);
 }
 
+// The same on small grids: a lane's column of eliminated rows stays in LDS
+// between the two sweeps of k_d0solve, LX columns a wavefront (the lanes past
+// them idle) so that it fits beside the coefficients.  v is read and dv/dy
+// written once as in k_dy_window, without its window's substitutions.
+// Bound by the row's chain and one wavefront's requests a CU: 63 x 128 x 63 34 us
+// (k_dy_window 59, the streamed sweep of k_d0solve 43), 40 x 257 x 40 60 us (104,
+// 76), 32 columns a wavefront there.
+template <int LX>
+__global__ void __launch_bounds__(64)
+    k_dy_lds(Dims D, D0Const fc, const double *__restrict__ f0, const double *__restrict__ der,
+             const double2 *__restrict__ src, double2 *__restrict__ dst, double sx, double sz) {
+  extern __shared__ double cfs[];
+  d0_rows_to_lds<64>(cfs, f0, der, D.ny);
+  const D0Rows<1> co{cfs, f0, der};
+  const int col = blockIdx.x * LX + threadIdx.x, m = D.ny, mi = m - 2;
+  if ((int)threadIdx.x >= LX || col >= D.ncol) return;
+  // row i at xr[i LX], behind the coefficients (D0C is even: 16-byte aligned)
+  double2 *const xr = (double2 *)(cfs + (size_t)m * D0C) + threadIdx.x;
+  int ix, iz;
+  col_ix_iz(D, col, ix, iz);
+  const size_t nc = D.ncol;
+  C x1, x2, sx0, sx1, r25, r27;
+  d0_forward<1, 1>(D, co, src, xr, LX, col, x1, x2, sx0, sx1, r25, r27);
+  const C ph = cexpi(-(D.alfa0 * ix * sx + D.beta0 * iz * sz));
+  C b1, b2;
+  d0_border(fc, ph, x1, x2, sx0, sx1, r25, r27, b1, b2);
+  const C cph = conj(ph);
+  const C yb1 = cph * b1, yb2 = cph * b2;
+  st(dst + (size_t)(m - 2 + 2) * nc + col, b1);
+  st(dst + (size_t)(m - 1 + 2) * nc + col, b2);
+  C xk1 = b1, xk2 = b2;
+  rows_descending<8, C>(
+      mi, [&](int i) { return ld(xr + i * LX); },
+      [&](int i, const C &x) {
+        const C xk = x - co.f(i, 5) * yb1 - co.f(i, 6) * yb2 - co.f(i, 3) * xk1 - co.f(i, 4) * xk2;
+        st(dst + (size_t)(i + 2) * nc + col, xk);
+        xk2 = xk1;
+        xk1 = xk;
+      });
+}
+
+// columns a wavefront of k_dy_lds on this grid, 0: not taken
+static int dy_lds_lanes(const Dims &D) {
+  for (int lx : {64, 32}) {
+    const size_t lds = d0_lds_bytes(D.ny) + (size_t)(D.ny - 2) * 16 * lx;
+    if (lds <= 160 * 1024 && D.ncol <= 256 * lx) return lx;
+  }
+  return 0;
+}
+
+// Where the one-sweep dv/dy is the faster: from LDS wherever that is taken, and
+// above some 30,000 columns, where bytes count; between them the streamed sweep
+// (85 x 147 x 91, 15,738 columns: 50 us against 68; 64 x 257 x 64: 75 against 105;
+// 128 x 257 x 128, 33,153 columns: 118 against 115).
+bool dy_one_sweep(const Dims &D) { return dy_lds_lanes(D) != 0 || D.ncol > 30000; }
+
 int launch_dy_window(const Dims &D, const double2 *src, double2 *dst, const double *f0rows, const D0Const &fc,
                      const double *der, const double *sig, double sx, double sz, hipStream_t s) {
   if (D.ny - 2 < 2 * DYW_N + DYW_W) return hipErrorInvalidValue;
+  if (const int lx = dy_lds_lanes(D)) {
+    const size_t lds = d0_lds_bytes(D.ny) + (size_t)(D.ny - 2) * 16 * lx;
+    if (lx == 64)
+      hipLaunchKernelGGL(k_dy_lds<64>, dim3((D.ncol + 63) / 64), dim3(64), lds, s, D, fc, f0rows, der, src, dst, sx, sz);
+    else
+      hipLaunchKernelGGL(k_dy_lds<32>, dim3((D.ncol + 31) / 32), dim3(64), lds, s, D, fc, f0rows, der, src, dst, sx, sz);
+    return hipGetLastError();
+  }
   dim3 grid((D.ncol + 255) / 256);
   const size_t lds = (size_t)(D.ny - 2) * DYC * sizeof(double);
   if (lds <= 65536)
@@ -1317,23 +1452,30 @@ int dy_window_rows() { return DYW_W; }
 // a column comes out with the same bits as through the whole-field solves.
 // ws: the workspace of ncols columns (U1, U2, B1, B2, XR of the untabled
 // sweep; XR only for D0 and DY).
-template <int K>
-__global__ void __launch_bounds__(256)
-    k_line_cols(Dims D, int col0, int ncols, double lam, const double *__restrict__ der,
+// CL: the rows' coefficients from a copy in LDS.
+template <int K, int CL>
+__global__ void __launch_bounds__(64)
+    k_line_cols(Dims D, int col0, int ncols, double lam, const double *__restrict__ derg,
                 const double *__restrict__ f0, D0Const fc, const double2 *__restrict__ src,
                 double2 *__restrict__ dst, PentaWS ws, double sx, double sz) {
-  const int l = blockIdx.x * blockDim.x + threadIdx.x;
+  extern __shared__ double cfs[];
+  constexpr bool D0K = K == KD0 || K == KDY;
+  if constexpr (CL && D0K) d0_rows_to_lds<64>(cfs, f0, derg, D.ny);
+  if constexpr (CL && !D0K) rows_to_lds<64>(cfs, derg, D.ny * 20);
+  const double *const der = CL && !D0K ? cfs : derg;
+  const int l = blockIdx.x * 64 + threadIdx.x;
   if (l >= ncols) return;
   int ix, iz;
   col_ix_iz(D, col0 + l, ix, iz);
   Dims Ds = D;
   Ds.ncol = ncols;  // the row stride of src, dst and ws
   Ds.ncs = ncols;
-  if constexpr (K == KD0 || K == KDY) {
+  if constexpr (D0K) {
+    const D0Rows<CL> co{cfs, f0, derg};
     const size_t nc = ncols;
     const int m = D.ny;
     C x1, x2, sx0, sx1, r25, r27;
-    d0_forward<K == KDY ? 1 : 0>(Ds, f0, der, src, ws.XR, l, x1, x2, sx0, sx1, r25, r27);
+    d0_forward<K == KDY ? 1 : 0, CL>(Ds, co, src, ws.XR + l, nc, l, x1, x2, sx0, sx1, r25, r27);
     const C ph = cexpi(-(D.alfa0 * ix * sx + D.beta0 * iz * sz));
     C b1, b2;
     d0_border(fc, ph, x1, x2, sx0, sx1, r25, r27, b1, b2);
@@ -1342,16 +1484,16 @@ __global__ void __launch_bounds__(256)
     st(dst + (size_t)(m - 2 + 2) * nc + l, b1);
     st(dst + (size_t)(m - 1 + 2) * nc + l, b2);
     C xk1 = b1, xk2 = b2;
-    rows_descending<PF_BWD, C>(
+    rows_descending<8, C>(
         m - 2, [&](int i) { return ld(ws.XR + (size_t)i * nc + l); },
         [&](int i, const C &xr) {
-          const C xk = xr - F0(i, 5) * yb1 - F0(i, 6) * yb2 - F0(i, 3) * xk1 - F0(i, 4) * xk2;
+          const C xk = xr - co.f(i, 5) * yb1 - co.f(i, 6) * yb2 - co.f(i, 3) * xk1 - co.f(i, 4) * xk2;
           st(dst + (size_t)(i + 2) * nc + l, xk);
           xk2 = xk1;
           xk1 = xk;
         });
   } else {
-    penta_line<K, false>(Ds, l, ix, iz, 0, lam, der, src, dst, ws, nullptr, sx, sz);
+    penta_line<K, false, 8, 8>(Ds, l, ix, iz, 0, lam, der, src, dst, ws, nullptr, sx, sz);
   }
 }
 
@@ -1376,9 +1518,13 @@ int launch_line_cols(const Dims &D, int kind, double lambda, int col0, int ncols
     pw.B1 = (double *)(w + rows * 32);
     pw.B2 = (double *)(w + rows * 40);
   }
-  dim3 grid((ncols + 255) / 256);
-#define L(K) hipLaunchKernelGGL((k_line_cols<K>), grid, dim3(256), 0, s, D, col0, ncols, lambda, der, f0rows, fc, src, \
-                                dst, pw, sx, sz)
+  dim3 grid((ncols + 63) / 64);
+  const size_t lds = (kind == KD0 || kind == KDY) ? d0_lds_bytes(D.ny) : (size_t)D.ny * 20 * sizeof(double);
+  const bool cl = lds <= 65536;
+#define L1(K, CLX)                                                                                                   \
+  hipLaunchKernelGGL((k_line_cols<K, CLX>), grid, dim3(64), CLX ? lds : 0, s, D, col0, ncols, lambda, der, f0rows, fc, \
+                     src, dst, pw, sx, sz)
+#define L(K) do { if (cl) L1(K, 1); else L1(K, 0); } while (0)
   switch (kind) {
     case KD2V: L(KD2V); break;
     case KETA: L(KETA); break;
@@ -1388,6 +1534,7 @@ int launch_line_cols(const Dims &D, int kind, double lambda, int col0, int ncols
     default: return hipErrorInvalidValue;
   }
 #undef L
+#undef L1
   return hipGetLastError();
 }
 
@@ -1544,11 +1691,12 @@ __device__ __forceinline__ void shift_column(const Dims &D, const D0Const &fc, Q
   st(q + (size_t)(0 + 2) * nc + col, acc);
 }
 
-__global__ void __launch_bounds__(256)
+template <int NT>
+__global__ void __launch_bounds__(NT)
     k_exact_shift(Dims D, D0Const fc, QList ql, const double *__restrict__ f0, const double *__restrict__ der,
                   const double2 *__restrict__ PX, const double2 *__restrict__ PZ, double sx0s, double sz0s,
                   double sx1s, double sz1s) {
-  const int col = blockIdx.x * blockDim.x + threadIdx.x;
+  const int col = blockIdx.x * NT + threadIdx.x;
   if (col >= D.ncol) return;
   const int k = blockIdx.y;
   // the checkpoints of array k in its XR buffer ((ny-2)/EXS_CHUNK + 1 rows of 32 B)
@@ -1564,8 +1712,12 @@ int launch_exact_shift(const Dims &D, int nq, void *const *q, const int *f32, do
                        const double2 *PZ, double sx0, double sz0, double sx1, double sz1, hipStream_t s) {
   QList ql;
   for (int k = 0; k < nq; k++) { ql.q[k] = q[k]; ql.xr[k] = XR[k]; ql.f32[k] = f32[k]; }
-  dim3 grid((D.ncol + 255) / 256, nq);
-  hipLaunchKernelGGL(k_exact_shift, grid, dim3(256), 0, s, D, fc, ql, f0rows, der, PX, PZ, sx0, sz0, sx1, sz1);
+  if (small_columns(D, nq))
+    hipLaunchKernelGGL(k_exact_shift<64>, dim3((D.ncol + 63) / 64, nq), dim3(64), 0, s, D, fc, ql, f0rows, der, PX, PZ,
+                       sx0, sz0, sx1, sz1);
+  else
+    hipLaunchKernelGGL(k_exact_shift<256>, dim3((D.ncol + 255) / 256, nq), dim3(256), 0, s, D, fc, ql, f0rows, der, PX,
+                       PZ, sx0, sz0, sx1, sz1);
   return hipGetLastError();
 }
 
@@ -1805,8 +1957,8 @@ __device__ __forceinline__ void shift_window_column(const Dims &D, const D0Const
   }
 }
 
-template <int CL>
-__global__ void __launch_bounds__(256, 2)
+template <int CL, int NT>
+__global__ void __launch_bounds__(NT, NT == 64 ? 1 : 2)
     k_shift_window(Dims D, D0Const fc, QList ql, const double *__restrict__ f0, const double *__restrict__ der,
                    const double *__restrict__ sig, const double2 *__restrict__ PX, const double2 *__restrict__ PZ,
                    double sx0s, double sz0s, double sx1s, double sz1s) {
@@ -1815,23 +1967,23 @@ __global__ void __launch_bounds__(256, 2)
   if constexpr (CL) {
     // [row j < m][SHC]: D0 taps -2..2, then F0 columns 0, 1, 2, 7, 8, 3, 4 (rows < mi)
     const int n = m * SHC;
-    for (int b0 = 0; b0 < n; b0 += 16 * 256) {
+    for (int b0 = 0; b0 < n; b0 += 16 * NT) {
       double v[16];
 #pragma unroll
       for (int u = 0; u < 16; u++) {
-        const int k = min(b0 + u * 256 + (int)threadIdx.x, n - 1), j = k / SHC, c = k - j * SHC;
+        const int k = min(b0 + u * NT + (int)threadIdx.x, n - 1), j = k / SHC, c = k - j * SHC;
         const int fj = c == 5 ? 0 : (c == 6 ? 1 : (c == 7 ? 2 : (c == 8 ? 7 : (c == 9 ? 8 : (c == 10 ? 3 : 4)))));
         v[u] = c < 5 ? DER(der, j, 0, c - 2) : (j < mi ? F0(j, fj) : 0.0);
       }
 #pragma unroll
       for (int u = 0; u < 16; u++) {
-        const int k = b0 + u * 256 + threadIdx.x;
+        const int k = b0 + u * NT + threadIdx.x;
         if (k < n) cfs[k] = v[u];
       }
     }
     __syncthreads();
   }
-  const int col = blockIdx.x * blockDim.x + threadIdx.x;
+  const int col = blockIdx.x * NT + threadIdx.x;
   if (col >= D.ncol) return;
   const int k = blockIdx.y;
   if (ql.f32[k])
@@ -1849,14 +2001,18 @@ int launch_shift_window(const Dims &D, int nq, void *const *q, const int *f32, d
   if (D.ny - 2 < 2 * SHW_N + SHW_W || nq < 1 || nq > 4) return hipErrorInvalidValue;
   QList ql;
   for (int k = 0; k < nq; k++) { ql.q[k] = q[k]; ql.xr[k] = XR[k]; ql.f32[k] = f32[k]; }
-  dim3 grid((D.ncol + 255) / 256, nq);
   const size_t lds = (size_t)D.ny * SHC * sizeof(double);
-  if (lds <= 65536)
-    hipLaunchKernelGGL(k_shift_window<1>, grid, dim3(256), lds, s, D, fc, ql, f0rows, der, sig, PX, PZ, sx0, sz0,
-                       sx1, sz1);
-  else
-    hipLaunchKernelGGL(k_shift_window<0>, grid, dim3(256), 0, s, D, fc, ql, f0rows, der, sig, PX, PZ, sx0, sz0, sx1,
-                       sz1);
+#define L(CL, NT)                                                                                                   \
+  hipLaunchKernelGGL((k_shift_window<CL, NT>), dim3((D.ncol + NT - 1) / NT, nq), dim3(NT), CL ? lds : 0, s, D, fc, ql, \
+                     f0rows, der, sig, PX, PZ, sx0, sz0, sx1, sz1)
+  // one wavefront a block takes all of a SIMD's registers (nothing spills then):
+  // while half of the SIMDs are left for the solves beside it, 64 x 128 x 64
+  // 128 -> 106 us, 85 x 147 x 91 133 -> 127; at 127 x 257 x 127 it takes them and the
+  // step is 6 % longer
+  const bool small = small_columns(D, 2 * nq);
+  if (lds <= 65536) { if (small) L(1, 64); else L(1, 256); }
+  else { if (small) L(0, 64); else L(0, 256); }
+#undef L
   return hipGetLastError();
 }
 
