@@ -1,10 +1,12 @@
 // Host-side set-up of libhstgpu: derived deck values, the y grid, the compact
 // weights, the seeded initial field and the column-independent factorisation
 // of the D0 matrix.  No HIP calls here: these entry points run without a GPU.
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstring>
 #include <string>
+#include <system_error>
 #include <vector>
 
 #include "hst_internal.h"
@@ -344,6 +346,55 @@ double initial_energy(const hst_deck &d) {
   double q2 = 0.0;
   for (double v : part) q2 += v;
   return q2;
+}
+
+// The threads of one transfer end with it and wait by yielding meanwhile (an
+// OpenMP team's spin on for a while, beside the caller's own).  The pieces are
+// taken from a counter, so that threads which get no processor hold nothing up.
+CopyTeam::CopyTeam() {
+  const int n = std::min(7, (int)std::thread::hardware_concurrency() - 1);
+  for (int w = 0; w < n; w++) {
+    try {
+      threads.emplace_back([this] {
+        while (!stop.load(std::memory_order_acquire))
+          if (!pieces()) std::this_thread::yield();
+      });
+    } catch (const std::system_error &) {
+      break;  // fewer threads
+    }
+  }
+}
+
+CopyTeam::~CopyTeam() {
+  stop.store(true, std::memory_order_release);
+  for (std::thread &t : threads) t.join();
+}
+
+// Copies pieces until none is left; false: there was none.  `next` passes PIECES
+// at the end of a copy and is set back, its arguments written, at the next one's
+// start: a thread that comes late finds no piece of either.
+bool CopyTeam::pieces() {
+  bool any = false;
+  while (next.load(std::memory_order_relaxed) < PIECES) {
+    const size_t k = next.fetch_add(1, std::memory_order_acq_rel);
+    if (k >= PIECES) break;
+    const size_t step = ((len + PIECES - 1) / PIECES + 4095) / 4096 * 4096;
+    const size_t a = std::min(len, k * step), b = std::min(len, a + step);
+    if (b > a) std::memcpy((char *)to + a, (const char *)from + a, b - a);
+    done.fetch_add(1, std::memory_order_release);
+    any = true;
+  }
+  return any;
+}
+
+void CopyTeam::copy(void *dst, const void *src, size_t n) {
+  to = dst;
+  from = src;
+  len = n;
+  done.store(0, std::memory_order_relaxed);
+  next.store(0, std::memory_order_release);
+  pieces();
+  while (done.load(std::memory_order_acquire) < PIECES) std::this_thread::yield();
 }
 
 Dims make_dims(const hst_deck &d, const hst_grid_info &g) {

@@ -3,10 +3,12 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <complex>
 #include <functional>
 #include <cstdint>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/hst_gpu.h"
@@ -238,6 +240,25 @@ int launch_product_to_field(const Dims &D, int mixed, const void *P, double2 *ds
 
 // ---------------------------------------------------------------- shared helpers
 
+// Copies between host buffers by up to eight threads, for the length of one
+// transfer: the pages of a fresh destination are then taken in parallel (one
+// thread fills them at 10 GB/s).
+class CopyTeam {
+ public:
+  CopyTeam();
+  ~CopyTeam();
+  void copy(void *dst, const void *src, size_t n);
+
+ private:
+  static constexpr size_t PIECES = 8;  // of 2 MB at a full copy: threads that meet in one huge page each fill it
+  bool pieces();
+  std::vector<std::thread> threads;
+  std::atomic<size_t> next{PIECES}, done{PIECES};
+  std::atomic<bool> stop{false};
+  void *to = nullptr;
+  const void *from = nullptr;
+  size_t len = 0;
+};
 Dims make_dims(const hst_deck &d, const hst_grid_info &g);
 D0Const d0_const(const D0Factor &f);
 // The shear shifts (sx, sz) of a deck at time t (src/hst_derivatives.f90:123-128).
