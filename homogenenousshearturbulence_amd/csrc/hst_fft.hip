@@ -487,19 +487,18 @@ struct XL {
 constexpr bool xline_size(int M) { return M % 3 == 0 ? M >= 24 : M >= 16; }
 
 // The x pass's radices: those of the z lines for M = 2^a; for M = 3 2^a the
-// radix 3 comes second, so that the first and the last stage divide E.
-__host__ __device__ constexpr int xl_rest(int R, int i) {  // radix i of the rest R after 8 and 3
-  return R == 16 ? 4 : R <= 8 ? R : (i == 0 ? 8 : R / 8);
-}
+// radix 3 (or 6) comes second, so that the first and the last stage divide E.
+// M = 384 takes 8, 6, 8: three stages in the place of 8, 3, 4, 4.
+__host__ __device__ constexpr int xl_second(int M) { return M == 384 ? 6 : 3; }
+__host__ __device__ constexpr int xl_first(int M) { return M == 24 ? 4 : 8; }
 __host__ __device__ constexpr int xl_radix(int M, int st) {
   if (M % 3) return radix_at(M, st);
-  const int first = M == 24 ? 4 : 8;
-  return st == 0 ? first : (st == 1 ? 3 : xl_rest(M / (3 * first), st - 2));
+  const int rest = M / (xl_first(M) * xl_second(M));
+  return st == 0 ? xl_first(M) : (st == 1 ? xl_second(M) : (rest <= 8 ? rest : (st == 2 ? 8 : rest / 8)));
 }
 __host__ __device__ constexpr int xl_stages(int M) {
   if (M % 3) return n_stages(M);
-  const int R = M / (M == 24 ? 12 : 24);
-  return 2 + (R > 8 ? 2 : 1);
+  return M / (xl_first(M) * xl_second(M)) > 8 ? 4 : 3;
 }
 
 __device__ __forceinline__ int padx(int p) { return p + (p >> 3); }
@@ -559,27 +558,28 @@ __device__ __forceinline__ void xl_fft(Cx<R> (&v)[XL<M>::E], Cx<R> *L, int t, bo
     constexpr int Ls = M / (S * RAD);
     constexpr bool FIRST = (S == 1), LAST = (S * RAD == M);
     constexpr int OFF = xtw_off<M>(ST);
-    if constexpr (RAD == 3) {
-      // M/3 butterflies, two for each of the line's TS = M/6 lanes
+    if constexpr (RAD % 3 == 0) {
+      // M/RAD butterflies, two (one) for each of the line's TS = M/6 lanes
       static_assert(!FIRST && !LAST && 6 * TS == M, "the radix-3 stage lies inside");
-      Cx<R> c[2][3];
+      constexpr int NB = 6 / RAD;
+      Cx<R> c[NB][RAD];
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NB; j++) {
         const int b = t + TS * j, q = b % S, n1 = b / S;
 #pragma unroll
-        for (int n2 = 0; n2 < 3; n2++) c[j][n2] = L[padx(q + S * (n1 + Ls * n2))];
+        for (int n2 = 0; n2 < RAD; n2++) c[j][n2] = L[padx(q + S * (n1 + Ls * n2))];
       }
       xl_sync<M>();
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NB; j++) {
         const int b = t + TS * j, q = b % S, n1 = b / S;
-        dft<R, SIGN, 3>(c[j]);
-        L[padx(q + S * 3 * n1)] = c[j][0];
+        dft<R, SIGN, RAD>(c[j]);
+        L[padx(q + S * RAD * n1)] = c[j][0];
 #pragma unroll
-        for (int k2 = 1; k2 < 3; k2++) {
+        for (int k2 = 1; k2 < RAD; k2++) {
           Cx<R> w = tw[OFF + (k2 - 1) * Ls + n1];
           if (SIGN > 0) w.y = -w.y;
-          L[padx(q + S * k2 + S * 3 * n1)] = c[j][k2] * w;
+          L[padx(q + S * k2 + S * RAD * n1)] = c[j][k2] * w;
         }
       }
       xl_sync<M>();

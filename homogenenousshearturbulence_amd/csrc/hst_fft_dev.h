@@ -80,6 +80,21 @@ __device__ __forceinline__ void dft4(Cx<R> *v) {
   v[3] = b - d;
 }
 
+// 6 = 2 x 3 without inner twiddles: x[3 n1 + 2 n2] through the three-point
+// transforms over n2, X[k] = A_0[k mod 3] + (-1)^k A_1[k mod 3]
+template <typename R, int SIGN>
+__device__ __forceinline__ void dft6(Cx<R> *v) {
+  Cx<R> a[3] = {v[0], v[2], v[4]}, b[3] = {v[3], v[5], v[1]};
+  dft3<R, SIGN>(a);
+  dft3<R, SIGN>(b);
+  v[0] = a[0] + b[0];
+  v[3] = a[0] - b[0];
+  v[4] = a[1] + b[1];
+  v[1] = a[1] - b[1];
+  v[2] = a[2] + b[2];
+  v[5] = a[2] - b[2];
+}
+
 template <typename R, int SIGN>
 __device__ __forceinline__ void dft8(Cx<R> *v) {
   const R r2 = (R)0.70710678118654752440;
@@ -109,6 +124,7 @@ __device__ __forceinline__ void dft(Cx<R> *v) {
   if constexpr (RAD == 2) dft2<R, SIGN>(v);
   else if constexpr (RAD == 3) dft3<R, SIGN>(v);
   else if constexpr (RAD == 4) dft4<R, SIGN>(v);
+  else if constexpr (RAD == 6) dft6<R, SIGN>(v);
   else dft8<R, SIGN>(v);
 }
 
