@@ -873,10 +873,18 @@ __global__ void __launch_bounds__(64)
   else penta_full_line<KETA>(D, col, ix, iz, g, lam, der, pa.src[1], pa.dst[1], pa.ws[1].XR, t, sx, sz);
 }
 
-// blockIdx.y selects the system: K0 for the first, K1 for the second
-template <int K0, int K1, bool TAB>
-__global__ void __launch_bounds__(256)
-    k_penta(Dims D, PentaArgs pa, double lam, const double *__restrict__ der, double sx, double sz) {
+// blockIdx.y selects the system: K0 for the first, K1 for the second.
+// CL: the stencil rows from a copy in LDS (ny <= 409), two wavefronts a block: as
+// scalar loads they were waited for row by row in both sweeps, which shows where
+// a SIMD has one wavefront.  128 x 257 x 128 343 -> 291 us (313 with four
+// wavefronts a block, 387 with one, for which the copies leave no room on the
+// CU), 192 x 257 x 192 651 -> 633, 256 x 385 x 256 1807 -> 1783.
+template <int K0, int K1, bool TAB, int CL, int NT>
+__global__ void __launch_bounds__(NT)
+    k_penta(Dims D, PentaArgs pa, double lam, const double *__restrict__ derg, double sx, double sz) {
+  extern __shared__ double ders[];
+  if constexpr (CL) rows_to_lds<NT>(ders, derg, D.ny * 20);
+  const double *const der = CL ? ders : derg;
   // with the factor tables the +iz and -iz columns share a wavefront (one
   // load of a table row serves both) and neighbouring blocks stay on one XCD
   const int l = TAB ? xcd_linear() : blockIdx.x + gridDim.x * blockIdx.y;
@@ -951,8 +959,17 @@ int launch_penta(const Dims &D, int nsys, const int *kinds, double lambda, const
     hipLaunchKernelGGL(k_penta_full, dim3(pair_lanes(D) / 64, 2), dim3(64), 0, s, D, pa, lambda, der, sx, sz);
     return hipGetLastError();
   }
-  dim3 grid(((tab ? pair_lanes(D) : D.ncol) + 255) / 256, nsys);
-#define L(A, B, T) hipLaunchKernelGGL((k_penta<A, B, T>), grid, dim3(256), 0, s, D, pa, lambda, der, sx, sz)
+  const size_t lds = (size_t)D.ny * 20 * sizeof(double);
+  const bool cl = lds <= 65536;
+  const int nt = cl ? 128 : 256;
+  dim3 grid(((tab ? pair_lanes(D) : D.ncol) + nt - 1) / nt, nsys);
+#define L(A, B, T)                                                                                         \
+  do {                                                                                                     \
+    if (cl)                                                                                                \
+      hipLaunchKernelGGL((k_penta<A, B, T, 1, 128>), grid, dim3(128), lds, s, D, pa, lambda, der, sx, sz); \
+    else                                                                                                   \
+      hipLaunchKernelGGL((k_penta<A, B, T, 0, 256>), grid, dim3(256), 0, s, D, pa, lambda, der, sx, sz);   \
+  } while (0)
   if (nsys == 2 && kinds[0] == KD2V && kinds[1] == KETA) {
     if (tab) L(KD2V, KETA, true); else L(KD2V, KETA, false);
   } else if (nsys == 1 && kinds[0] == KD2V) L(KD2V, KD2V, false);
