@@ -2310,11 +2310,20 @@ int launch_ghosts(const Dims &D, int nf, double2 *const *f, double sx, double sz
 // The first reduction of outstats (src/hst_stats.f90:153-198): per block the
 // NSTAT sums uu vv ww uv vw uw eps mfx mfz q_in q_out e_in e_out ed pd
 // ncol_damped; the column energies of the spectrum on the way (:224-238).
-__global__ void __launch_bounds__(256)
+// G parts of the rows (wavefronts of one block).  With one part the grid has 73
+// blocks at 96 x 193 x 96, each walking all of its rows; with four 152 -> 65 us
+// there, and outstats as a whole 128 x 257 x 128 0.569 -> 0.472 ms.  Above 65,536
+// columns one part already fills the chip, and four are slower (outstats 256 x 257
+// x 256 1.49 against 1.53 ms).
+constexpr int ST_C = 256;
+template <int ST_G>
+__global__ void __launch_bounds__(ST_G *ST_C)
     k_stats(Dims D, StatsArgs a, const double2 *__restrict__ V1, const double2 *__restrict__ V2,
             const double2 *__restrict__ V3, const double *__restrict__ dyl, double *__restrict__ part,
             double *__restrict__ exz) {
-  const int col = blockIdx.x * blockDim.x + threadIdx.x;
+  const int part_of = threadIdx.x / ST_C, col = blockIdx.x * ST_C + threadIdx.x % ST_C;
+  const int iy0 = (int)((long long)D.ny * part_of / ST_G), iy1 = (int)((long long)D.ny * (part_of + 1) / ST_G);
+  __shared__ double qcs[ST_G][ST_C];
   double s[NSTAT];
 #pragma unroll
   for (int k = 0; k < NSTAT; k++) s[k] = 0.0;
@@ -2324,10 +2333,10 @@ __global__ void __launch_bounds__(256)
     const double al = D.alfa0 * ix, be = D.beta0 * iz, kk = al * al + be * be;
     const size_t nc = D.ncol;
     const double gd = a.gdamp ? a.gdamp[col] : 0.0;
-    if (gd > 0.0) s[15] = 1.0;
+    if (gd > 0.0 && part_of == 0) s[15] = 1.0;
     // the column energy sum_y w |u|^2 of the spectrum, every column
     double qc = 0.0;
-    for (int iy = 0; iy < D.ny; iy++) {
+    for (int iy = iy0; iy < iy1; iy++) {
       const size_t o = (size_t)(iy + 2) * nc + col;
       const C cu = ld(V1 + o), cv = ld(V2 + o), cw = ld(V3 + o);
       const double dy = dyl[iy];
@@ -2369,9 +2378,9 @@ __global__ void __launch_bounds__(256)
         s[12] += w * kk * (uu + vv + wv);
       }
     }
-    if (exz) exz[col] += qc;
+    qcs[part_of][threadIdx.x % ST_C] = qc;
   }
-  __shared__ double red[4][NSTAT];
+  __shared__ double red[ST_G * ST_C / 64][NSTAT];
 #pragma unroll
   for (int k = 0; k < NSTAT; k++) {
     double v = s[k];
@@ -2381,15 +2390,25 @@ __global__ void __launch_bounds__(256)
   __syncthreads();
   if (threadIdx.x < NSTAT) {
     const int k = threadIdx.x;
-    part[(size_t)blockIdx.x * NSTAT + k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
+    double v = 0.0;
+    for (int w = 0; w < ST_G * ST_C / 64; w++) v += red[w][k];
+    part[(size_t)blockIdx.x * NSTAT + k] = v;
+  }
+  if (exz && part_of == 0 && col < D.ncol) {
+    double qc = 0.0;
+    for (int g = 0; g < ST_G; g++) qc += qcs[g][threadIdx.x];
+    exz[col] += qc;
   }
 }
 
 int launch_stats(const Dims &D, const StatsArgs &a, const double2 *V1, const double2 *V2, const double2 *V3,
                  const double *dyl, double *part, int *n_part, double *exz_acc, hipStream_t s) {
-  dim3 grid((D.ncol + 255) / 256);
+  dim3 grid((D.ncol + ST_C - 1) / ST_C);
   if (n_part) *n_part = grid.x;
-  hipLaunchKernelGGL(k_stats, grid, dim3(256), 0, s, D, a, V1, V2, V3, dyl, part, exz_acc);
+  if (small_columns(D, 1))
+    hipLaunchKernelGGL(k_stats<4>, grid, dim3(4 * ST_C), 0, s, D, a, V1, V2, V3, dyl, part, exz_acc);
+  else
+    hipLaunchKernelGGL(k_stats<1>, grid, dim3(ST_C), 0, s, D, a, V1, V2, V3, dyl, part, exz_acc);
   return hipGetLastError();
 }
 
@@ -2513,8 +2532,12 @@ int launch_damping_mask(const Dims &D, int mixed, const double *gdamp, double2 *
 // src/hst_pressure.f90:35-88):
 //   D0 [alfa^2 uu + beta^2 ww + 2 alfa beta uw] - D2 vv - 2 i alfa D1 uv
 //   - 2 i beta D1 vw - 2 i (S alfa + S2 beta) D0 v,
-// the (0,0) column -<vv>, the raw product.  Stencils of the products in PR.
-template <typename PR>
+// the (0,0) column -<vv>, the raw product.  The seven fields of a row are first
+// put together, in FP64, into the three that the stencils take (D0, D1 and D2),
+// and a lane keeps five rows of those: each row of a field is read (RC + 4) / RC
+// times, not five (96 x 193 x 96 in FP64 267 -> 120 us, bound by HBM).  16 rows a
+// lane where the grid makes 512 blocks that way, 4 below.
+template <typename PR, int RC>
 __global__ void __launch_bounds__(256)
     k_pressure_rhs(Dims D, const typename PTraits<PR>::T2 *__restrict__ P0, size_t pstride,
                    const double2 *__restrict__ V2, double2 *__restrict__ R, const double *__restrict__ der,
@@ -2524,40 +2547,52 @@ __global__ void __launch_bounds__(256)
   int ix, iz;
   col_ix_iz(D, col, ix, iz);
   const double al = D.alfa0 * ix, be = D.beta0 * iz;
+  const double aa = al * al, bb = be * be, ab = 2.0 * al * be, sv = 2.0 * (D.S * al + s2now * be);
   const bool m00 = (ix == 0 && iz == 0);
   const size_t nc = D.ncol;
-  const int iy = blockIdx.y;
-  auto sten = [&](int q, int n) {
-    Cx<PR> a{0, 0};
+  const int i0 = blockIdx.y * RC;
+  C a[5], b[5], c[5];  // rows i - 2 .. i + 2 under D0, under D1, under D2
+  auto push = [&](int row) {
+    const size_t o = (size_t)(row + 2) * nc + col;
+    auto P = [&](int q) {
+      const Cx<PR> z = ldp<PR>(P0 + q * pstride + o);
+      return C{(double)z.x, (double)z.y};
+    };
 #pragma unroll
-    for (int j = -2; j <= 2; j++) a = a + (PR)DER(der, iy, n, j) * ldp<PR>(P0 + q * pstride + (size_t)(iy + j + 2) * nc + col);
-    return C{(double)a.x, (double)a.y};
+    for (int k = 0; k < 4; k++) { a[k] = a[k + 1]; b[k] = b[k + 1]; c[k] = c[k + 1]; }
+    a[4] = aa * P(0) + bb * P(2) + ab * P(5) - imul(sv, ld(V2 + o));
+    b[4] = imul(2.0 * al, P(3)) + imul(2.0 * be, P(4));
+    c[4] = P(1);
   };
-  C d0v{0, 0};
 #pragma unroll
-  for (int j = -2; j <= 2; j++) d0v = d0v + DER(der, iy, 0, j) * ld(V2 + (size_t)(iy + j + 2) * nc + col);
-  C r = (al * al) * sten(0, 0) - imul(2.0 * (D.S * al + s2now * be), d0v);
-  r = r - sten(1, 2);
-  if (m00) {
-    const Cx<PR> vv = ldp<PR>(P0 + 1 * pstride + (size_t)(iy + 2) * nc + col);
-    r = C{-(double)vv.x, 0.0};
+  for (int k = -2; k < 2; k++) push(i0 + k);
+#pragma unroll 4
+  for (int k = 0; k < RC; k++) {
+    const int i = i0 + k;
+    if (i >= D.ny) break;
+    push(i + 2);
+    C r{0, 0};
+#pragma unroll
+    for (int j = 0; j < 5; j++)
+      r = r + DER(der, i, 0, j - 2) * a[j] - DER(der, i, 1, j - 2) * b[j] - DER(der, i, 2, j - 2) * c[j];
+    if (m00) r = C{-c[2].x, 0.0};
+    st(R + (size_t)(i + 2) * nc + col, r);
   }
-  r = r + (be * be) * sten(2, 0);
-  r = r - imul(2.0 * al, sten(3, 1));
-  r = r - imul(2.0 * be, sten(4, 1));
-  r = r + (2.0 * al * be) * sten(5, 0);
-  st(R + (size_t)(iy + 2) * nc + col, r);
 }
 
 int launch_pressure_rhs(const Dims &D, int mixed, const void *P0, const double2 *V2, double2 *R, const double *der,
                         double s2now, hipStream_t s) {
-  dim3 grid((D.ncol + 255) / 256, D.ny);
   const size_t pstride = (size_t)D.NYg * D.ncol;
-  if (mixed)
-    hipLaunchKernelGGL(k_pressure_rhs<float>, grid, dim3(256), 0, s, D, (const float2 *)P0, pstride, V2, R, der, s2now);
-  else
-    hipLaunchKernelGGL(k_pressure_rhs<double>, grid, dim3(256), 0, s, D, (const double2 *)P0, pstride, V2, R, der,
-                       s2now);
+  const int nb = (D.ncol + 255) / 256;
+#define L(PR, T2, RC)                                                                                             \
+  hipLaunchKernelGGL((k_pressure_rhs<PR, RC>), dim3(nb, (D.ny + RC - 1) / RC), dim3(256), 0, s, D, (const T2 *)P0, \
+                     pstride, V2, R, der, s2now)
+  if ((long long)nb * D.ny >= 512 * 16) {
+    if (mixed) L(float, float2, 16); else L(double, double2, 16);
+  } else {
+    if (mixed) L(float, float2, 4); else L(double, double2, 4);
+  }
+#undef L
   return hipGetLastError();
 }
 
