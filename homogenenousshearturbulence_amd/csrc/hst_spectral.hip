@@ -907,8 +907,9 @@ __global__ void __launch_bounds__(NT)
 // the 64 B a row and column of the sweeps, and saves the pivots' chains: below
 // some 24,000 columns (375 wavefronts a system) those chains bound the solve,
 // above it the bytes.  k_penta with checkpoints -> k_penta_full, us: 32 x 65 x 32
-// 55 -> 22, 63 x 128 x 63 125 -> 52, 64 x 257 x 64 268 -> 110, 95 x 64 x 95 (18,336
-// columns) 69 -> 50, 128 x 257 x 128 (33,153) 361 -> 402.  The fused shift and
+// 55 -> 22, 63 x 128 x 63 125 -> 52, 64 x 257 x 64 268 -> 110 and, with the
+// checkpoints' stencil rows in LDS, 95 x 64 x 95 (18,336 columns) 59 -> 50, 108 x
+// 193 x 108 (23,653) 171 -> 164, 128 x 257 x 128 (33,153) 291 -> 402.  The fused shift and
 // solve, whose chain is the longer: 32 x 65 x 32 86 -> 43, 64 x 128 x 64 209 -> 111,
 // 127 x 257 x 127 (32,640 columns) 575 -> 397, 160 x 200 x 160 (51,681) 519 -> 557.
 bool penta_full_tables(const Dims &D) { return D.ncol <= (D.exact ? 33000 : 24000); }
