@@ -61,7 +61,7 @@ struct State {
   size_t part_cap = 0;
   double *h_part = nullptr;  // pinned host copy of d_part (the CFL maxima of a time step)
   int n_part_pending = 0;
-  char *h_stage = nullptr;  // two pinned pieces of STAGE_BYTES for the downloads
+  char *h_stage = nullptr;  // two pinned pieces of STAGE_BYTES for the transfers of host arrays
   hipEvent_t ev_stage[2] = {nullptr, nullptr};
   double2 *F[9] = {nullptr};
   void *P = nullptr, *Hv = nullptr, *Hp = nullptr, *ws = nullptr;

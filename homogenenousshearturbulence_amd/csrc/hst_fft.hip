@@ -2,13 +2,14 @@
 //
 //   k_zift   z inverse transform of u, v, w (3/2 padding fused into the load),
 //            written transposed to x-fastest lines (Hv)
-//   k_xpass  per (row, z point): x inverse real transform of u, v, w, the six
+//   k_xline  per (row, z point): x inverse real transform of u, v, w, the six
 //            products (and the CFL number), x forward real transforms of the
-//            products truncated to the nx+1 kept modes (Hp)
+//            products truncated to the nx+1 kept modes (Hp); k_xpass the same
+//            for the shortest lines
 //   k_zfft   z forward transform of the six products, truncated to the 2nz+1
 //            kept modes, written to the spectral layout (P)
 //
-// Every transform is an in-LDS Stockham FFT of radices 8, 4, 2 and 3 with the
+// Every transform is an in-LDS Stockham FFT of radices 8, 6, 4, 3 and 2 with the
 // butterflies held in registers between the two barriers of a stage.  Real
 // transforms of length 2M run as complex transforms of length M.  Field
 // layout on the device: [row][ix][iz] with iz fastest (a Fourier column is

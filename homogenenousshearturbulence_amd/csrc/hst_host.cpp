@@ -359,7 +359,7 @@ CopyTeam::CopyTeam() {
         while (!stop.load(std::memory_order_acquire))
           if (!pieces()) std::this_thread::yield();
       });
-    } catch (const std::system_error &) {
+    } catch (const std::exception &) {
       break;  // fewer threads
     }
   }
