@@ -75,6 +75,8 @@ struct State {
   double ptab_lam[3] = {0.0, 0.0, 0.0};
   int ptab_next = 0;
   bool ptab_off = false;
+  int64_t ptab_bytes = 0;        // the tables held
+  size_t ptab_limit = SIZE_MAX;  // their most (HST_TABLES_MB)
   void *tables = nullptr;
   hipStream_t stream = nullptr;
   // the oldrhs half of the exact shift runs on a second stream, beside the
@@ -527,23 +529,46 @@ static int ghosts(int nf, double2 *const *f, double sx, double sz) {
   return run("ghosts", nf * 8.0 * S.D.ncol * 16.0, [&] { return launch_ghosts(S.D, nf, f, sx, sz, S.stream); });
 }
 
+static void drop_tables() {
+  for (int k = 0; k < 3; k++) {
+    for (void *&p : S.ptab[k]) {
+      if (p) (void)hipFree(p);  // (waits for the solves that read it)
+      p = nullptr;
+    }
+    S.ptab_lam[k] = 0.0;
+  }
+  S.bytes_held -= S.ptab_bytes;
+  S.ptab_bytes = 0;
+}
+
 // Memory for the factor tables of slot k, or false (and no tables from then
-// on) when they do not fit.
+// on) when they do not fit beside 4 GB left free, or into HST_TABLES_MB.  Where
+// the whole factorisation does not fit (72 B a row and group, in each of the six
+// tables) all slots go over to checkpoints, a ninth of that.
 static bool penta_slot(int k) {
   if (S.ptab[k][0]) return true;
   const size_t tb = penta_table_bytes(S.D);
   size_t free_b = 0, total_b = 0;
-  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < 2 * tb + ((size_t)4 << 30)) {
+  bool ok = hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b >= 2 * tb + ((size_t)4 << 30) &&
+            (size_t)S.ptab_bytes + 2 * tb <= S.ptab_limit;
+  for (int j = 0; j < 2 && ok; j++) ok = hipMalloc(&S.ptab[k][j], tb) == hipSuccess;
+  if (ok) {
+    S.ptab_bytes += 2 * (int64_t)tb;
+    S.bytes_held += 2 * (int64_t)tb;
+    return true;
+  }
+  (void)hipGetLastError();
+  for (void *&p : S.ptab[k]) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+  }
+  if (!S.D.full) {
     S.ptab_off = true;
     return false;
   }
-  if (hipMalloc(&S.ptab[k][0], tb) != hipSuccess || hipMalloc(&S.ptab[k][1], tb) != hipSuccess) {
-    (void)hipGetLastError();
-    S.ptab_off = true;
-    return false;
-  }
-  S.bytes_held += 2 * (int64_t)tb;
-  return true;
+  drop_tables();
+  S.D.full = 0;
+  return penta_slot(k);
 }
 
 // the main stream waits for factor tables under way on the side stream
@@ -568,9 +593,13 @@ static int penta_prebuild(double deltat) {
     have = have && found;
   }
   if (have) return 0;
+  for (int full = -1; full != S.D.full;) {  // (again, if the slots went over to checkpoints)
+    full = S.D.full;
+    for (int k = 0; k < 3; k++)
+      if (!penta_slot(k)) return 0;
+  }
   void *tabs[6];
   for (int k = 0; k < 3; k++) {
-    if (!penta_slot(k)) return 0;
     tabs[2 * k] = S.ptab[k][0];
     tabs[2 * k + 1] = S.ptab[k][1];
     S.ptab_lam[k] = 0.0;  // (no lambda, if the launch fails)
@@ -581,9 +610,11 @@ static int penta_prebuild(double deltat) {
     HIPCHK(hipEventRecord(S.ev_fork, S.stream));
     HIPCHK(hipStreamWaitEvent(S.side, S.ev_fork, 0));
   }
-  if (int rc = run_on(st, "penta_factor", 6.0 * (double)penta_table_bytes(S.D),
-                      [&] { return launch_penta_factor(S.D, 3, lam, tabs, S.d_der, st); }))
-    return rc;
+  if (run_on(st, "penta_factor", 6.0 * (double)penta_table_bytes(S.D),
+             [&] { return launch_penta_factor(S.D, 3, lam, tabs, S.d_der, st); })) {
+    S.ptab_off = true;
+    return 0;
+  }
   if (!serial) {
     HIPCHK(hipEventRecord(S.ev_tab, S.side));
     S.tab_pending = true;
@@ -849,6 +880,7 @@ int hst_gpu_init(const hst_deck *deck, int precision) {
   if (!fft_size_supported(S.g.nxd)) return fail("unsupported x transform size nxd = " + std::to_string(S.g.nxd));
   S.D = make_dims(*deck, S.g);
   Dims &D = S.D;
+  D.full = penta_full_tables(D, deck->exact_shift) ? 1 : 0;
   d0_factor(S.der, D.ny, S.f0);
   S.fc = d0_const(S.f0);
   {
@@ -875,6 +907,8 @@ int hst_gpu_init(const hst_deck *deck, int precision) {
   // device memory): the exact shift of rhs runs apart from the line solves,
   // which eliminate their rows through the full workspace
   if (const char *e = std::getenv("HST_NO_TABLES")) S.ptab_off = std::atoi(e) != 0;
+  // HST_TABLES_MB: the most device memory that the factor tables take
+  if (const char *e = std::getenv("HST_TABLES_MB")) S.ptab_limit = (size_t)std::max(std::atoll(e), 0LL) << 20;
   const size_t nf = (size_t)D.NYg * D.ncol;
   const size_t cs = S.mixed ? sizeof(float2) : sizeof(double2);
   int64_t held = 0;

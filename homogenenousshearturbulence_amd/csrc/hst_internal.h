@@ -42,7 +42,7 @@ struct Dims {
   // columns, so that every row starts on a 4 KB boundary (column sweeps over
   // such rows measured 7-10 % faster than over rows 16 B off the lines)
   int ncs;
-  int exact;  // the deck's exact_shift
+  int full;  // the factor tables hold the whole factorisation (1) or checkpoints (0)
   double alfa0, beta0, ni, S, factor, dx, dz;
 };
 
@@ -112,9 +112,10 @@ int launch_penta(const Dims &D, int nsys, const int *kinds, double lambda, const
                  double sz, hipStream_t s);
 // The matrix part of the D2V and ETA lines for each of nlam lambdas (tabs: D2V,
 // ETA of the first, of the second, ..; penta_table_bytes of device memory each):
-// per (ix, |iz|) group the whole factorisation where penta_full_tables says so,
-// else its state every 8 rows, from which the solves recompute the rows.
-bool penta_full_tables(const Dims &D);
+// per (ix, |iz|) group the whole factorisation (D.full), else its state every 8
+// rows, from which the solves recompute the rows.  penta_full_tables: whether the
+// whole factorisation is the faster on this grid, where it fits.
+bool penta_full_tables(const Dims &D, bool exact_shift);
 size_t penta_table_bytes(const Dims &D);
 int launch_penta_factor(const Dims &D, int nlam, const double *lambda, void *const *tabs, const double *der,
                         hipStream_t s);

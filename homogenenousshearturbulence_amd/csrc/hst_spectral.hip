@@ -912,11 +912,11 @@ __global__ void __launch_bounds__(NT)
 // 193 x 108 (23,653) 171 -> 164, 128 x 257 x 128 (33,153) 291 -> 402.  The fused shift and
 // solve, whose chain is the longer: 32 x 65 x 32 86 -> 43, 64 x 128 x 64 209 -> 111,
 // 127 x 257 x 127 (32,640 columns) 575 -> 397, 160 x 200 x 160 (51,681) 519 -> 557.
-bool penta_full_tables(const Dims &D) { return D.ncol <= (D.exact ? 33000 : 24000); }
+bool penta_full_tables(const Dims &D, bool exact_shift) { return D.ncol <= (exact_shift ? 33000 : 24000); }
 
 size_t penta_table_bytes(const Dims &D) {
   const size_t ng = (size_t)(D.nx + 1) * (D.nz + 1);
-  if (penta_full_tables(D)) return penta_full_bytes(D.ny - 2, ng);
+  if (D.full) return penta_full_bytes(D.ny - 2, ng);
   return (size_t)2 * ((D.ny - 2 + PC - 1) / PC) * ng * sizeof(double4);
 }
 
@@ -934,7 +934,7 @@ int launch_penta_factor(const Dims &D, int nlam, const double *lambda, void *con
   const size_t lds = (size_t)D.ny * 20 * sizeof(double);
   const bool cl = lds <= 65536;
 #define L(F, CLX) hipLaunchKernelGGL((k_penta_factor<F, CLX>), grid, dim3(64), CLX ? lds : 0, s, D, a, der)
-  if (penta_full_tables(D)) {
+  if (D.full) {
     if (cl) L(true, 1); else L(true, 0);
   } else {
     if (cl) L(false, 1); else L(false, 0);
@@ -955,7 +955,7 @@ int launch_penta(const Dims &D, int nsys, const int *kinds, double lambda, const
     pa.tab[k] = tabs ? tabs[k] : nullptr;
     if (!pa.tab[k]) tab = false;
   }
-  if (tab && penta_full_tables(D)) {
+  if (tab && D.full) {
     if (nsys != 2 || kinds[0] != KD2V || kinds[1] != KETA) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_penta_full, dim3(pair_lanes(D) / 64, 2), dim3(64), 0, s, D, pa, lambda, der, sx, sz);
     return hipGetLastError();
@@ -2264,7 +2264,7 @@ int launch_shift_penta(const Dims &D, const double2 *q2, const double2 *q1, doub
 #define L(CLX, F, NT)                                                                                             \
   hipLaunchKernelGGL((k_shift_penta<CLX, F, NT>), dim3((D.ncol + NT - 1) / NT, 2), dim3(NT), CLX ? lds : 0, s, D, a, \
                      fcr, f0r, der, PX, PZ, sx0, sz0, sx1, sz1, lambda)
-  if (penta_full_tables(D)) {
+  if (D.full) {
     if (lds <= 49152) L(1, true, 64); else L(0, true, 64);
   } else {
     if (lds <= 49152) L(1, false, 256); else L(0, false, 256);
