@@ -909,10 +909,18 @@ __global__ void __launch_bounds__(NT)
 // above it the bytes.  k_penta with checkpoints -> k_penta_full, us: 32 x 65 x 32
 // 55 -> 22, 63 x 128 x 63 125 -> 52, 64 x 257 x 64 268 -> 110 and, with the
 // checkpoints' stencil rows in LDS, 95 x 64 x 95 (18,336 columns) 59 -> 50, 108 x
-// 193 x 108 (23,653) 171 -> 164, 128 x 257 x 128 (33,153) 291 -> 402.  The fused shift and
-// solve, whose chain is the longer: 32 x 65 x 32 86 -> 43, 64 x 128 x 64 209 -> 111,
-// 127 x 257 x 127 (32,640 columns) 575 -> 397, 160 x 200 x 160 (51,681) 519 -> 557.
-bool penta_full_tables(const Dims &D, bool exact_shift) { return D.ncol <= (exact_shift ? 33000 : 24000); }
+// 193 x 108 (23,653) 171 -> 164, 128 x 257 x 128 (33,153) 291 -> 402.  The fused
+// shift and solve, whose chain is the longer, takes it while its blocks of one
+// wavefront, which have a SIMD's registers to themselves, find a SIMD each: 32 x 65
+// x 32 86 -> 43, 64 x 128 x 64 209 -> 111, 127 x 257 x 127 (32,640 columns, 1020
+// blocks) 570 -> 397; past that line a second round of blocks makes it no faster,
+// 127 x 257 x 128 (32,896 columns, 1028 blocks) 580 -> 580 and 127 x 129 x 128 280
+// -> 281, and the step, whose tables are larger, longer: 6.56-6.72 -> 6.80-6.82 ms
+// and 3.49-3.57 -> 3.60 ms.
+constexpr int SIMDS = 1024;  // 256 CUs of four
+bool penta_full_tables(const Dims &D, bool exact_shift) {
+  return exact_shift ? 2 * ((D.ncol + 63) / 64) <= SIMDS : D.ncol <= 24000;
+}
 
 size_t penta_table_bytes(const Dims &D) {
   const size_t ng = (size_t)(D.nx + 1) * (D.nz + 1);
@@ -1179,7 +1187,7 @@ __global__ void __launch_bounds__(NT)
 // A column kernel's block: one wavefront where nsys systems of the grid's columns
 // make fewer wavefronts than the chip has SIMDs (each then has a CU's caches, LDS
 // and memory path nearly to itself), four above.
-static bool small_columns(const Dims &D, int nsys) { return (long long)D.ncol * nsys <= 64 * 1024; }
+static bool small_columns(const Dims &D, int nsys) { return (long long)D.ncol * nsys <= 64 * SIMDS; }
 
 int launch_d0solve(const Dims &D, int rhs_mode, int out_mode, int nf, const double2 *const *src, double2 *const *dst,
                    double2 *dst3, double2 *const *XR, const double *f0rows, const D0Const &fc, const double *der,

@@ -53,6 +53,32 @@ def test_tables_that_fit(oracle_built, monkeypatch, limit, held, exact):
         assert rel(V[c][..., 2:-2], o.V[c][..., 2:-2]) <= 1e-11, c
 
 
+# with the exact shift the whole factorisation up to 1024 blocks of 64 columns and
+# system: 32,640, 32,767 (the last block not full) and 32,896 columns
+@pytest.mark.parametrize("nx,nz,whole", [(127, 127, True), (216, 75, True), (127, 128, False)])
+def test_column_line(oracle_built, nx, nz, whole):
+    ny = 9
+    d = dataclasses.replace(read_input(deck_path("small")), nx=nx, ny=ny, nz=nz, exact_shift=True, kpeak=2.0)
+    o = oracle_built.Oracle(d)
+    o.initial_field()
+    o.fill_all_ghosts(0.0)
+    s = hst.Solver(d, hst.FP64)
+    try:
+        s.set_V(o.V)
+        s.reset_old()
+        s.fill_all_ghosts(0.0)
+        before = s.memory()[0]
+        o.timestep(1e-3)
+        s.timestep(1e-3)
+        groups = (nx + 1) * (nz + 1)
+        assert s.memory()[0] - before == 6 * groups * (((ny - 2) * 9 + 17) * 8 if whole else 2 * 32)
+        V = s.V
+    finally:
+        s.close()
+    for c in range(3):
+        assert rel(V[c][..., 2:-2], o.V[c][..., 2:-2]) <= 1e-11, c
+
+
 @pytest.mark.parametrize("exact", [False, True])
 def test_pieces_that_run_out(monkeypatch, exact):
     """A pair of whole tables a solve, of which the second goes over to
