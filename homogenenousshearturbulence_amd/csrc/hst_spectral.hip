@@ -1440,11 +1440,19 @@ static int dy_lds_lanes(const Dims &D) {
   return 0;
 }
 
-// Where the one-sweep dv/dy is the faster: from LDS wherever that is taken, and
-// above some 30,000 columns, where bytes count; between them the streamed sweep
-// (85 x 147 x 91, 15,738 columns: 50 us against 68; 64 x 257 x 64: 75 against 105;
-// 128 x 257 x 128, 33,153 columns: 118 against 115).
-bool dy_one_sweep(const Dims &D) { return dy_lds_lanes(D) != 0 || D.ncol > 30000; }
+// Where the one-sweep dv/dy is the faster: from LDS wherever that is taken, above
+// some 30,000 columns, where bytes count, and where the streamed sweep is held up:
+// lines whose coefficients do not fit LDS (ny > 585: 64 x 641 x 64 434 us streamed
+// against 236, 64 x 1025 x 64 710 against 570), and grids whose v and eliminated
+// rows, written and read back, do not fit the 256 MB cache together (95 x 513 x 95
+// 202 against 196, 121 x 401 x 121 172 against 162).  Between them the streamed
+// sweep (64 x 257 x 64 75 us against 105, 85 x 513 x 85 178 against 194, 104 x 257 x
+// 104 99 against 106, 121 x 129 x 121 56 against 65; 122 x 129 x 122, 30,135
+// columns, 65 either way).
+bool dy_one_sweep(const Dims &D) {
+  const bool cached = (long long)D.ncol * D.ny * 2 * 16 <= 256ll << 20;
+  return dy_lds_lanes(D) != 0 || D.ncol > 30000 || !cached || d0_lds_bytes(D.ny) > 65536;
+}
 
 int launch_dy_window(const Dims &D, const double2 *src, double2 *dst, const double *f0rows, const D0Const &fc,
                      const double *der, const double *sig, double sx, double sz, hipStream_t s) {
