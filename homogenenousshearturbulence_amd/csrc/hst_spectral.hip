@@ -10,6 +10,8 @@
 // cache.  Every kernel with a recurrence in y runs one column per lane.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "hst_cx.h"
 #include "hst_internal.h"
 
@@ -874,11 +876,19 @@ __global__ void __launch_bounds__(64)
 }
 
 // blockIdx.y selects the system: K0 for the first, K1 for the second.
-// CL: the stencil rows from a copy in LDS (ny <= 409), two wavefronts a block: as
-// scalar loads they were waited for row by row in both sweeps, which shows where
-// a SIMD has one wavefront.  128 x 257 x 128 343 -> 291 us (313 with four
-// wavefronts a block, 387 with one, for which the copies leave no room on the
-// CU), 192 x 257 x 192 651 -> 633, 256 x 385 x 256 1807 -> 1783.
+// CL: the stencil rows from a copy in LDS (ny <= 409).  As scalar loads they are
+// waited for row by row in both sweeps, which shows where a SIMD has one wavefront;
+// the copy in turn limits the blocks a CU holds.  Blocks of two wavefronts share one
+// while all of them are resident at once, three a CU or what LDS holds; above that
+// the lines with tables take it four wavefronts a block, and those without, which
+// stream their rows, leave it.  D2V and ETA with tables, us (no copy, four wavefronts
+// | copy, two | copy, four): 128 x 257 x 128 345 | 297 | 316, 150 x 257 x 150 385 |
+// 339 | 369, 128 x 409 x 128 (two blocks a CU) 553 | 602 | 508, 165 x 257 x 165 415 |
+// 512 | 401, 200 x 129 x 200 310 | 338 | 313, 230 x 257 x 230 930 | 908 | 870, 300 x
+// 257 x 300 1552 | 1523 | 1479; at 180 x 257 x 180, where the wavefronts make two a
+// SIMD exactly, 470 | 582 | 497.  Poisson without tables: 128 x 257 x 128 312 | 288 |
+// 274, 200 x 257 x 200 696 | 657 | 683, 230 x 257 x 230 779 | 952 | 787, 300 x 257 x
+// 300 1370 | 1550 | 1421.
 template <int K0, int K1, bool TAB, int CL, int NT>
 __global__ void __launch_bounds__(NT)
     k_penta(Dims D, PentaArgs pa, double lam, const double *__restrict__ derg, double sx, double sz) {
@@ -917,7 +927,8 @@ __global__ void __launch_bounds__(NT)
 // 127 x 257 x 128 (32,896 columns, 1028 blocks) 580 -> 580 and 127 x 129 x 128 280
 // -> 281, and the step, whose tables are larger, longer: 6.56-6.72 -> 6.80-6.82 ms
 // and 3.49-3.57 -> 3.60 ms.
-constexpr int SIMDS = 1024;  // 256 CUs of four
+constexpr int CUS = 256, SIMDS = 4 * CUS;
+constexpr size_t LDS_BYTES = 160 * 1024;  // of a CU
 bool penta_full_tables(const Dims &D, bool exact_shift) {
   return exact_shift ? 2 * ((D.ncol + 63) / 64) <= SIMDS : D.ncol <= 24000;
 }
@@ -969,15 +980,17 @@ int launch_penta(const Dims &D, int nsys, const int *kinds, double lambda, const
     return hipGetLastError();
   }
   const size_t lds = (size_t)D.ny * 20 * sizeof(double);
-  const bool cl = lds <= 65536;
-  const int nt = cl ? 128 : 256;
-  dim3 grid(((tab ? pair_lanes(D) : D.ncol) + nt - 1) / nt, nsys);
-#define L(A, B, T)                                                                                         \
-  do {                                                                                                     \
-    if (cl)                                                                                                \
-      hipLaunchKernelGGL((k_penta<A, B, T, 1, 128>), grid, dim3(128), lds, s, D, pa, lambda, der, sx, sz); \
-    else                                                                                                   \
-      hipLaunchKernelGGL((k_penta<A, B, T, 0, 256>), grid, dim3(256), 0, s, D, pa, lambda, der, sx, sz);   \
+  const int lanes = tab ? pair_lanes(D) : D.ncol;
+  const int resident = CUS * (int)std::min<size_t>(3, LDS_BYTES / lds);
+  const bool two = lds <= 65536 && nsys * ((lanes + 127) / 128) <= resident;
+#define L1(A, B, T, CL, NT)                                                                                   \
+  hipLaunchKernelGGL((k_penta<A, B, T, CL, NT>), dim3((lanes + NT - 1) / NT, nsys), dim3(NT), CL ? lds : 0, s, D, \
+                     pa, lambda, der, sx, sz)
+#define L(A, B, T)                                          \
+  do {                                                      \
+    if (two) L1(A, B, T, 1, 128);                           \
+    else if (T && lds <= 65536) L1(A, B, T, (T ? 1 : 0), 256); \
+    else L1(A, B, T, 0, 256);                               \
   } while (0)
   if (nsys == 2 && kinds[0] == KD2V && kinds[1] == KETA) {
     if (tab) L(KD2V, KETA, true); else L(KD2V, KETA, false);
@@ -986,6 +999,7 @@ int launch_penta(const Dims &D, int nsys, const int *kinds, double lambda, const
   else if (nsys == 1 && kinds[0] == KPOISSON) L(KPOISSON, KPOISSON, false);
   else return hipErrorInvalidValue;
 #undef L
+#undef L1
   return hipGetLastError();
 }
 
