@@ -1214,10 +1214,19 @@ int launch_d0solve(const Dims &D, int rhs_mode, int out_mode, int nf, const doub
     fl.dst[k] = dst ? dst[k] : nullptr;
     fl.XR[k] = XR[k];
   }
-  const bool small = small_columns(D, nf);
-  const int nt = small ? 64 : 256;
+  // One wavefront a block while all blocks are resident (four a CU, or what LDS
+  // holds; three without the copy), four above; the copy of the coefficients while
+  // there are no more wavefronts than SIMDs: it limits the blocks a CU holds, and from
+  // there on is the slower.  dv/dy with u, w, us (no copy, four wavefronts | copy,
+  // four | copy, one): 128 x 257 x 128 275 | 213 | 185, 165 x 257 x 165 298 | 259 | 297,
+  // 165 x 409 x 165 (859 blocks, three a CU) 488 | 425 | 581, 180 x 409 x 180 537 | 521 |
+  // 688, 200 x 257 x 200 491 | 529 | 441, 256 x 257 x 256 753 | 812 | 754, 256 x 409 x
+  // 256 1237 | 1340 | 1196, 300 x 257 x 300 1015 | 1049 | 1124.
   const size_t lds = d0_lds_bytes(D.ny);
-  const bool cl = lds <= 65536;
+  const bool cl = lds <= 65536 && small_columns(D, nf);
+  const int per_cu = cl ? (int)std::min<size_t>(4, LDS_BYTES / lds) : 3;
+  const bool small = small_columns(D, nf) && nf * ((D.ncol + 63) / 64) <= CUS * per_cu;
+  const int nt = small ? 64 : 256;
   dim3 grid((D.ncol + nt - 1) / nt, nf);
   if (n_part) *n_part = grid.x * grid.y;
 #define L4(R, O, CLX, NT)                                                                                        \
