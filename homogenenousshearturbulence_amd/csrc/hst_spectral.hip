@@ -61,7 +61,7 @@ __device__ __forceinline__ Cx<PR> ldp(const typename PTraits<PR>::T2 *p) {
 // 1, 2: add the products of group 1 or 2 to rhs, oldrhs as buildrhs(ODE, g);
 // 4: prepare and the five combined products of the x pass's MODE 3
 // (vv - uu, vv - ww, uv, vw, uw), the same sums regrouped.
-constexpr int RHS_ROWS = 16;  // the most rows of a chunk
+constexpr int RHS_ROWS = 64;  // the most rows of a chunk
 template <typename PR, int MODE, bool SHIFT>
 __global__ void __launch_bounds__(256)
     k_buildrhs(Dims D, RhsArgs a, const double2 *__restrict__ V1, const double2 *__restrict__ V2,
@@ -284,12 +284,20 @@ int launch_buildrhs(const Dims &D, int mixed, const RhsArgs &a, const double2 *V
   // CU, 8 down to one and a half blocks a CU, 4 and 2 below.  Against 64 rows
   // throughout, us (FP64, mixed): 32 x 65 x 32 130, 96 -> 15.5, 13.5 (4 rows);
   // 63 x 128 x 63 146, 108 -> 48, 35 (8); 128 x 257 x 128 508, 349 -> 377, 262
-  // (8; 16: 407, 271); 256 x 513 x 256 3057, 1970 -> 3102, 1850 (16; 8: 3086,
-  // 1903).  Running a column block's chunks side by side on one XCD, so that the
-  // shared rows meet in its L2, is 10 % slower (128 x 257 x 128: 420, 312).
+  // (8; 16: 407, 271); 256 x 513 x 256 3078, 1978 -> 3153, 1849 (16; 8: 3163,
+  // 1893).  A chunk's shared rows are read again a chunk of rows later; where 16
+  // rows of the fields read (v, eta and five products) exceed the 256 MB cache they
+  // come from HBM, and long chunks are the faster: 300 x 257 x 300 FP64 (20 MB a row)
+  // 2298 us in 16 rows, 2223 in 64, 300 x 700 x 300 5282, 4877, 512 x 513 x 512 11687,
+  // 10601, mixed 400 x 513 x 400 (23 MB) 5016, 4927, 512 x 1025 x 512 17444, 16287;
+  // below it the short ones, 256 x 257 x 256 FP64 (15 MB) 1517, 1570, mixed 340 x 257 x
+  // 340 (17 MB) 1780, 1887.  Running a column block's chunks side by side on one XCD,
+  // so that the shared rows meet in its L2, is 10 % slower (128 x 257 x 128: 420, 312).
   const int gx = (D.ncol + 255) / 256;
   auto blocks = [&](int r) { return (long long)gx * ((D.ny + r - 1) / r); };
-  const int rch = blocks(16) >= 4096 ? 16 : (blocks(8) >= 400 ? 8 : (blocks(4) >= 128 ? 4 : 2));
+  const bool cached = 16ll * D.ncol * (2 * 16 + 5 * (mixed ? 8 : 16)) <= 256ll << 20;
+  const int rch = !cached ? RHS_ROWS
+                          : (blocks(16) >= 4096 ? 16 : (blocks(8) >= 400 ? 8 : (blocks(4) >= 128 ? 4 : 2)));
   dim3 grid(gx, (D.ny + rch - 1) / rch);
   const size_t pstride = (size_t)D.NYg * D.ncol;
   // 0 prepare, 1/2 one group, 3 all, 4 all from the five combinations, 5 as 4
