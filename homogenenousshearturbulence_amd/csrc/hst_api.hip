@@ -1087,6 +1087,7 @@ static int to_device(void *dev, const void *host, size_t bytes) {
 int hst_gpu_upload_field(int field, const double *host) {
   if (int rc = check_live()) return rc;
   if (int rc = check_field(field)) return rc;
+  if (!host) return fail("upload_field: host is NULL");
   const size_t nf = (size_t)S.D.NYg * S.D.ncol;
   double2 *stage = (double2 *)S.ws, *wide = stage + nf;
   if (int rc = to_device(stage, host, nf * sizeof(double2))) return rc;
@@ -1100,6 +1101,7 @@ int hst_gpu_upload_field(int field, const double *host) {
 int hst_gpu_download_field(int field, double *host) {
   if (int rc = check_live()) return rc;
   if (int rc = check_field(field)) return rc;
+  if (!host) return fail("download_field: host is NULL");
   const size_t nf = (size_t)S.D.NYg * S.D.ncol;
   double2 *stage = (double2 *)S.ws, *wide = stage + nf;
   int rc = 0;

@@ -1,0 +1,32 @@
+"""Field transfers of other host memory than an ordinary array, on both sides of the
+sizes from which several threads copy (16 MiB down, 48 MiB up)."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from conftest import deck_path
+from homogenenousshearturbulence_amd import hst
+from homogenenousshearturbulence_amd.deck import read_input
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(3, 12, 3), (127, 478, 8), (63, 401, 69)]  # 7 kB, 16 MiB + 4 KB, 54 MiB
+
+
+def solver(nx, ny, nz):
+    return hst.Solver(dataclasses.replace(read_input(deck_path("small")), nx=nx, ny=ny, nz=nz), hst.FP64)
+
+
+@pytest.mark.parametrize("nx,ny,nz", SIZES)
+def test_null_is_refused(nx, ny, nz):
+    s = solver(nx, ny, nz)
+    try:
+        f = np.random.default_rng(1).standard_normal(s.shape) + 0j
+        s.upload(hst.V1, f)
+        for call in (hst.lib().hst_gpu_upload_field, hst.lib().hst_gpu_download_field):
+            assert call(hst.V1, None) != 0
+            assert "NULL" in hst.last_error()
+        assert np.array_equal(s.download(hst.V1), f)
+    finally:
+        s.close()
