@@ -348,16 +348,28 @@ double initial_energy(const hst_deck &d) {
   return q2;
 }
 
-// The threads of one transfer end with it and wait by yielding meanwhile (an
-// OpenMP team's spin on for a while, beside the caller's own).  The pieces are
-// taken from a counter, so that threads which get no processor hold nothing up.
+// The threads of one transfer end with it.  Between its pieces they wait by yielding
+// for a moment (the bus brings a piece in 0.3 ms; an OpenMP team's spin on for a
+// while after it, beside the caller's own), and sleep when it takes longer, as when
+// the transfer has to wait for work that is queued before it.  The pieces are taken
+// from a counter, so that threads which get no processor hold nothing up.
 CopyTeam::CopyTeam() {
   const int n = std::min(7, (int)std::thread::hardware_concurrency() - 1);
   for (int w = 0; w < n; w++) {
     try {
       threads.emplace_back([this] {
-        while (!stop.load(std::memory_order_acquire))
-          if (!pieces()) std::this_thread::yield();
+        int idle = 0;
+        while (!stop.load(std::memory_order_acquire)) {
+          if (pieces()) idle = 0;
+          else if (++idle < YIELDS) std::this_thread::yield();
+          else {
+            std::unique_lock<std::mutex> lk(mutex);
+            more.wait(lk, [this] {
+              return stop.load(std::memory_order_acquire) || next.load(std::memory_order_acquire) < PIECES;
+            });
+            idle = 0;
+          }
+        }
       });
     } catch (const std::exception &) {
       break;  // fewer threads
@@ -365,8 +377,15 @@ CopyTeam::CopyTeam() {
   }
 }
 
+// (taking the lock once orders the change before or after a thread's look at it)
+void CopyTeam::wake() {
+  { std::lock_guard<std::mutex> lk(mutex); }
+  more.notify_all();
+}
+
 CopyTeam::~CopyTeam() {
   stop.store(true, std::memory_order_release);
+  wake();
   for (std::thread &t : threads) t.join();
 }
 
@@ -393,6 +412,7 @@ void CopyTeam::copy(void *dst, const void *src, size_t n) {
   len = n;
   done.store(0, std::memory_order_relaxed);
   next.store(0, std::memory_order_release);
+  wake();
   pieces();
   while (done.load(std::memory_order_acquire) < PIECES) std::this_thread::yield();
 }

@@ -5,8 +5,10 @@
 
 #include <atomic>
 #include <complex>
+#include <condition_variable>
 #include <functional>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -252,13 +254,17 @@ class CopyTeam {
 
  private:
   static constexpr size_t PIECES = 8;  // of 2 MB at a full copy: threads that meet in one huge page each fill it
+  static constexpr int YIELDS = 512;
   bool pieces();
-  std::vector<std::thread> threads;
+  void wake();
+  std::mutex mutex;
+  std::condition_variable more;
   std::atomic<size_t> next{PIECES}, done{PIECES};
   std::atomic<bool> stop{false};
   void *to = nullptr;
   const void *from = nullptr;
   size_t len = 0;
+  std::vector<std::thread> threads;  // (the last member: they use the others)
 };
 Dims make_dims(const hst_deck &d, const hst_grid_info &g);
 D0Const d0_const(const D0Factor &f);

@@ -1,6 +1,7 @@
 """Field transfers of other host memory than an ordinary array, on both sides of the
 sizes from which several threads copy (16 MiB down, 48 MiB up)."""
 import dataclasses
+import time
 
 import numpy as np
 import pytest
@@ -28,5 +29,33 @@ def test_null_is_refused(nx, ny, nz):
             assert call(hst.V1, None) != 0
             assert "NULL" in hst.last_error()
         assert np.array_equal(s.download(hst.V1), f)
+    finally:
+        s.close()
+
+
+def cpu_share(call):
+    """The processors that a call keeps busy on average."""
+    c, w = time.process_time(), time.perf_counter()
+    call()
+    c, w = time.process_time() - c, time.perf_counter() - w
+    return c / w, w
+
+
+def test_waiting_for_queued_steps_is_idle():
+    """Steps queued, then a transfer that has to wait for them: of the copying
+    threads none is busy meanwhile (the caller's own wait is)."""
+    d = dataclasses.replace(read_input(deck_path("small")), nx=127, ny=257, nz=127)
+    s = hst.Solver(d, hst.FP64)
+    try:
+        f = np.zeros(s.shape, dtype=np.complex128)
+        s.download(hst.V1)
+        s.timestep(1e-4)
+        for call in (lambda: s.download(hst.V1), lambda: s.upload(hst.V1, f)):
+            s.sync()
+            for _ in range(120):
+                s.timestep(1e-4)
+            share, wall = cpu_share(call)
+            assert wall > 0.1  # (the queue was not empty)
+            assert share < 2.0
     finally:
         s.close()
