@@ -1035,6 +1035,17 @@ int hst_gpu_grid(hst_grid_info *info, double *y, double *dyl, double *der) {
   return 0;
 }
 
+// Ordinary memory of the caller's, which the bus does not reach by itself; pinned and
+// managed arrays go straight to hipMemcpy (54 MB through the pieces 1.05 -> 1.3 ms).
+static bool pageable(const void *host) {
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, host) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return at.type == hipMemoryTypeUnregistered;
+}
+
 // Between device memory and the caller's (pageable) buffers in two pinned pieces by
 // turns: while one is on the bus the team copies the other.  hipMemcpy stages such
 // buffers through one thread, at the rate at which it fills fresh pages on the way
@@ -1043,7 +1054,7 @@ int hst_gpu_grid(hst_grid_info *info, double *y, double *dyl, double *der) {
 // Downloads below a piece and uploads below three, whose pages one thread reads as
 // fast as they go, keep hipMemcpy (the threads cost as much as they save).
 static int to_host(void *host, const void *dev, size_t bytes) {
-  if (bytes < STAGE_BYTES) {
+  if (bytes < STAGE_BYTES || !pageable(host)) {
     HIPCHK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, S.stream));
     HIPCHK(hipStreamSynchronize(S.stream));
     return 0;
@@ -1067,7 +1078,7 @@ static int to_host(void *host, const void *dev, size_t bytes) {
 }
 
 static int to_device(void *dev, const void *host, size_t bytes) {
-  if (bytes < 3 * STAGE_BYTES) {
+  if (bytes < 3 * STAGE_BYTES || !pageable(host)) {
     HIPCHK(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, S.stream));
     return 0;
   }

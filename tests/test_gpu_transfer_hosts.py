@@ -5,6 +5,7 @@ import time
 
 import numpy as np
 import pytest
+import torch  # (first: its HIP runtime has to be the one in the process)
 
 from conftest import deck_path
 from homogenenousshearturbulence_amd import hst
@@ -57,5 +58,26 @@ def test_waiting_for_queued_steps_is_idle():
             share, wall = cpu_share(call)
             assert wall > 0.1  # (the queue was not empty)
             assert share < 2.0
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz", SIZES)
+def test_pinned_arrays_go_straight(nx, ny, nz):
+    """The caller's pinned arrays come back the same, at one processor's cost."""
+    s = solver(nx, ny, nz)
+    try:
+        a = torch.randn(s.shape + (2,), dtype=torch.float64, pin_memory=True)
+        b = torch.zeros(s.shape + (2,), dtype=torch.float64, pin_memory=True)
+        up, down = hst.lib().hst_gpu_upload_field, hst.lib().hst_gpu_download_field
+
+        def there_and_back():
+            for _ in range(20):
+                assert up(hst.V1, a.data_ptr()) == 0 and down(hst.V1, b.data_ptr()) == 0
+
+        there_and_back()
+        share, _ = cpu_share(there_and_back)
+        assert torch.equal(a, b)
+        assert share < 2.0
     finally:
         s.close()
