@@ -106,3 +106,26 @@ def test_pieces_that_run_out(monkeypatch, exact):
         out.append(got)
     for a, b in zip(*out):
         assert rel(b, a) <= 1e-11
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(20, 18, 9), (40, 130, 30)])
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("precision", [hst.FP64, hst.MIXED])
+def test_tables_beside_the_transforms(monkeypatch, nx, ny, nz, exact, precision):
+    """The tables of a changing step length, built on the second stream beside the
+    transforms, give the same bits as on the main stream (HST_SERIAL=1)."""
+    d = dataclasses.replace(read_input(deck_path("small")), nx=nx, ny=ny, nz=nz, exact_shift=exact, kpeak=2.0)
+    out = []
+    for serial in ("0", "1"):
+        monkeypatch.setenv("HST_SERIAL", serial)
+        s = hst.Solver(d, precision)
+        try:
+            s.initial_field()
+            s.reset_old()
+            s.fill_all_ghosts(0.0)
+            for k in range(12):
+                s.timestep(1e-3 * (1.0 + 0.1 * (k % 5)))
+            out.append(s.V)
+        finally:
+            s.close()
+    assert np.array_equal(out[0], out[1])
