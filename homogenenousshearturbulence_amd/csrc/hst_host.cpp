@@ -2,6 +2,7 @@
 // weights, the seeded initial field and the column-independent factorisation
 // of the D0 matrix.  No HIP calls here: these entry points run without a GPU.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <complex>
 #include <cstring>
@@ -349,25 +350,28 @@ double initial_energy(const hst_deck &d) {
 }
 
 // The threads of one transfer end with it.  Between its pieces they wait by yielding
-// for a moment (the bus brings a piece in 0.3 ms; an OpenMP team's spin on for a
+// for two milliseconds (the bus brings a piece in 0.3; an OpenMP team's spin on for a
 // while after it, beside the caller's own), and sleep when it takes longer, as when
-// the transfer has to wait for work that is queued before it.  The pieces are taken
-// from a counter, so that threads which get no processor hold nothing up.
+// the transfer has to wait for work that is queued before it.  Asleep within a piece's
+// time they are late for the next: 63 x 128 x 63, a download of two pieces, 1 % of a
+// 20-step job.  The pieces are taken from a counter, so that threads which get no
+// processor hold nothing up.
 CopyTeam::CopyTeam() {
   const int n = std::min(7, (int)std::thread::hardware_concurrency() - 1);
   for (int w = 0; w < n; w++) {
     try {
       threads.emplace_back([this] {
-        int idle = 0;
+        typedef std::chrono::steady_clock clock;
+        clock::time_point last = clock::now();
         while (!stop.load(std::memory_order_acquire)) {
-          if (pieces()) idle = 0;
-          else if (++idle < YIELDS) std::this_thread::yield();
+          if (pieces()) last = clock::now();
+          else if (clock::now() - last < std::chrono::milliseconds(2)) std::this_thread::yield();
           else {
             std::unique_lock<std::mutex> lk(mutex);
             more.wait(lk, [this] {
               return stop.load(std::memory_order_acquire) || next.load(std::memory_order_acquire) < PIECES;
             });
-            idle = 0;
+            last = clock::now();
           }
         }
       });

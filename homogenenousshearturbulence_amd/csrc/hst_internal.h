@@ -254,7 +254,6 @@ class CopyTeam {
 
  private:
   static constexpr size_t PIECES = 8;  // of 2 MB at a full copy: threads that meet in one huge page each fill it
-  static constexpr int YIELDS = 512;
   bool pieces();
   void wake();
   std::mutex mutex;
