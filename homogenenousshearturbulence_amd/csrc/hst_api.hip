@@ -59,7 +59,8 @@ struct State {
   D0Const fcr;
   double *d_f0r = nullptr;
   size_t part_cap = 0;
-  double *h_part = nullptr;  // pinned host copy of d_part (the CFL maxima of a time step)
+  // pinned host copy of d_part: the CFL maxima of a time step, the sums of outstats
+  double *h_part = nullptr;
   int n_part_pending = 0;
   char *h_stage = nullptr;  // two pinned pieces of STAGE_BYTES for the transfers of host arrays
   hipEvent_t ev_stage[2] = {nullptr, nullptr};
@@ -69,8 +70,8 @@ struct State {
   int chunk = 0;
   PentaWS pws[2];
   double2 *XR[4];
-  // factor tables of the D2V and ETA lines for up to three lambdas (the RK3
-  // substeps at a fixed step), built on first use when memory allows
+  // factor tables of the D2V and ETA lines for up to three lambdas: a time step's,
+  // built at its start where they are not held, or those of linsolve calls
   void *ptab[3][2] = {{nullptr, nullptr}, {nullptr, nullptr}, {nullptr, nullptr}};
   double ptab_lam[3] = {0.0, 0.0, 0.0};
   int ptab_next = 0;
@@ -102,8 +103,10 @@ struct State {
   int64_t bytes_held = 0;
   bool prof = false;
   bool serial = false;  // the oldrhs shift on the main stream (HST_SERIAL=1)
-  // the time step's dv/dy in one sweep (k_dy_window) when the D0 factor decays
-  // fast enough on this grid; HST_NO_DYWIN=1: the stored sweep of k_d0solve
+  // the time step's dv/dy in one sweep (k_dy_lds, k_dy_window) when the D0 factor
+  // decays fast enough on this grid (k_dy_lds does not need it to, but is asked for
+  // under the same condition) and that is the faster; else, or with HST_NO_DYWIN=1,
+  // the stored sweep of k_d0solve
   bool dyw = false;
   double *d_sig = nullptr;
   // the exact shift of oldrhs in one sweep (k_shift_window) under the same

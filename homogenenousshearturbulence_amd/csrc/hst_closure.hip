@@ -319,10 +319,10 @@ __device__ __forceinline__ void to_operands(const f4 h[4], bf8 B[2]) {
 // continued fraction, 7e-11 off at one, written as a correction to x); above,
 // +-1 -+ 2 / (exp(2 |x|) + 1), |x| cut at 10 where the correction is 4e-9.  One
 // reciprocal serves both, and since the correction is at most 0.24 of what it corrects
-// (31 % of the result, at one) its rounding hardly shows: over 4 M arguments of 1e-8 .. 12 the largest
-// error against 64 bits is 1.33 units of the last place and the rms 0.238
-// (tanhf: 1.35 and 0.240).  A wavefront evaluates 32 a tile, most of the
-// network's instructions: k_mlp_infer 116 -> 90 us on 798,720 points.
+// (31 % of the result, at one) its rounding hardly shows: over 4 M arguments of
+// 1e-8 .. 12 the largest error against 64 bits is 1.33 units of the last place and
+// the rms 0.238 (tanhf: 1.35 and 0.240).  A wavefront evaluates 32 a tile, most of
+// the network's instructions: k_mlp_infer 116 -> 90 us on 798,720 points.
 __device__ __forceinline__ float tanh_f(float x) {
   const float a = fabsf(x), c = a > 10.0f ? 10.0f : a, x2 = x * x;
   const bool small = a < 1.0f;

@@ -994,11 +994,11 @@ int launch_penta(const Dims &D, int nsys, const int *kinds, double lambda, const
 #define L1(A, B, T, CL, NT)                                                                                   \
   hipLaunchKernelGGL((k_penta<A, B, T, CL, NT>), dim3((lanes + NT - 1) / NT, nsys), dim3(NT), CL ? lds : 0, s, D, \
                      pa, lambda, der, sx, sz)
-#define L(A, B, T)                                          \
-  do {                                                      \
-    if (two) L1(A, B, T, 1, 128);                           \
+#define L(A, B, T)                                             \
+  do {                                                         \
+    if (two) L1(A, B, T, 1, 128);                              \
     else if (T && lds <= 65536) L1(A, B, T, (T ? 1 : 0), 256); \
-    else L1(A, B, T, 0, 256);                               \
+    else L1(A, B, T, 0, 256);                                  \
   } while (0)
   if (nsys == 2 && kinds[0] == KD2V && kinds[1] == KETA) {
     if (tab) L(KD2V, KETA, true); else L(KD2V, KETA, false);
